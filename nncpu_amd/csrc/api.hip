@@ -238,8 +238,10 @@ int run_gemv(const nnh_weight* w, const float* x, size_t x_stride, float* y, siz
                               y_stride, st);
     } else if (act == NNH_ACT_F32) {
         float* xsum = w->dtype == NNH_Q4S ? (float*)scratch : nullptr;
-        nnh::launch_gemv_f32(w->dtype, w->fq, w->fs, w->bi, x, x_stride, xsum, rows, nb, (int)w->nbp, (int)n_tok,
-                             y, y_stride, w->f32v2, st);
+        if (!nnh::launch_gemm_f32(w->dtype, w->qs, w->fs, w->bi, x, x_stride, xsum, rows, nb, (int)w->nbp,
+                                  (int)n_tok, y, y_stride, w->f32v2, st))
+            nnh::launch_gemv_f32(w->dtype, w->fq, w->fs, w->bi, x, x_stride, xsum, rows, nb, (int)w->nbp, (int)n_tok,
+                                 y, y_stride, w->f32v2, st);
     } else if (!(act == NNH_ACT_I8 && n_tok == 1 &&
                  nnh::launch_gemv_i8_qx(w->dtype, w->qs, w->sc, w->sb, x, rows, nb, y, st))) {
         // (One vector at most rows: quantized in the GEMV's own prologue.)

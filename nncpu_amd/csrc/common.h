@@ -116,8 +116,8 @@ void launch_relayout_f32(int dtype, const uint8_t* raw_qs, const uint16_t* raw_s
                          int rows, int nb, int nbp, bool v2, hipStream_t st);
 // Q4 block sums of n_tok vectors (kernels/scalar.rs:355-359 tree).
 void launch_block_sums(const float* x, size_t x_stride, int nb, int n_tok, float* xsum, hipStream_t st);
-// Bit-exact f32 gemv for n_tok <= 16 vectors; for Q4, xsum is scratch of
-// n_tok * nb floats (the block sums of x).
+// Bit-exact f32 gemv; for Q4, xsum is scratch of n_tok * nb floats (the block
+// sums of x).
 // One vector through the 8-lane (tall) kernel, y written and each
 // workgroup's largest argmax key into part[0..f32_v2_parts(rows)).
 int f32_v2_parts(int rows);
@@ -148,6 +148,14 @@ void launch_rmsnorm_vec(const NormIn& nrm, int cols, float* out, hipStream_t st)
 void launch_gemv_f32(int dtype, const uint8_t* fq, const uint16_t* fs, const uint16_t* biases, const float* x,
                      size_t x_stride, float* xsum, int rows, int nb, int nbp, int n_tok, float* y,
                      size_t y_stride, bool v2, hipStream_t st);
+
+// The same for several vectors on the f32 matrix unit (kernels_f32_batch.hip);
+// qs: the split layout's quants. False (nothing launched) for the few vectors
+// that launch_gemv_f32 takes faster, when x's rows are not 16-byte aligned or
+// an offset would not fit 32 bits.
+bool launch_gemm_f32(int dtype, const uint8_t* qs, const uint16_t* fs, const uint16_t* biases, const float* x,
+                     size_t x_stride, float* xsum, int rows, int nb, int nbp, int n_tok, float* y, size_t y_stride,
+                     bool v2, hipStream_t st);
 
 // int8 path (kernels_i8.hip).
 void launch_quantize_act(const float* x, size_t x_stride, int cols, int n_tok, int8_t* q, uint16_t* s, double* sx,

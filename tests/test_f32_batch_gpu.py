@@ -1,0 +1,65 @@
+"""The bit-exact f32 matmul of several vectors on the f32 matrix unit, against
+the oracle: every output bit, at the edges of its tiles (16 rows, 16 vectors,
+token tiles of up to 64), of its stages (8 blocks, steps of 4) and of Q4's
+bias groups (8 blocks), with strided rows, and with signed zeros, denormals,
+infinities and values whose products under- and overflow."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+N = pytest.importorskip("nncpu_amd")
+
+
+@pytest.fixture(scope="module", autouse=True)
+def device():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    N.init(0)
+
+
+def run(oracle, dtype, rows, cols, n_tok, pad=0, x=None, seed=0xB47C):
+    rng = oracle.Rng(seed + rows + cols + n_tok)
+    m = oracle.QMatrix.from_f32(dtype, rng.normals(rows * cols, 0.02).reshape(rows, cols))
+    w = N.Weight.from_split(dtype, m.buf, rows, cols)
+    xs, ys = cols + pad, rows + pad
+    if x is None:
+        x = rng.normals(n_tok * xs, 1.0)
+    y = np.full(n_tok * ys, 7.0, np.float32)
+    N.gemv_batch(w, x, xs, y, ys, n_tok, N.ACT_F32)
+    ref = np.full(n_tok * ys, 7.0, np.float32)
+    o = oracle.gemv_batch(m, x, n_tok, xs, ys, backend="avx2")
+    for t in range(n_tok):
+        ref[t * ys:t * ys + rows] = o[t * ys:t * ys + rows]
+    w.free()
+    return y, ref
+
+
+@pytest.mark.parametrize("dtype", [1, 2])
+@pytest.mark.parametrize("rows,cols,n_tok,pad", [
+    (1, 32, 5, 0), (15, 96, 16, 0), (16, 128, 17, 4), (17, 224, 6, 0), (33, 256, 32, 12), (40, 288, 33, 0),
+    (31, 1152, 49, 0), (70, 1184, 64, 4), (129, 608, 65, 0), (257, 992, 80, 8), (4100, 2080, 7, 0), (4112, 512, 40, 0),
+    (8200, 512, 81, 4), (12290, 544, 20, 0), (16400, 96, 130, 0), (100, 320, 9, 3),
+])
+def test_f32_batch_bit_exact(oracle, dtype, rows, cols, n_tok, pad):
+    y, ref = run(oracle, dtype, rows, cols, n_tok, pad)
+    assert np.array_equal(y.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("dtype", [1, 2])
+@pytest.mark.parametrize("cols", [288, 1024, 1184])
+def test_f32_batch_special_values(oracle, dtype, cols):
+    n_tok = 19
+    rng = np.random.default_rng(cols + dtype)
+    x = np.ldexp(rng.standard_normal(n_tok * cols), rng.integers(-150, 100, n_tok * cols)).astype(np.float32)
+    x[rng.integers(0, x.size, x.size // 4)] = 0.0
+    x[rng.integers(0, x.size, x.size // 4)] = -0.0
+    x.reshape(n_tok, cols)[3] = -0.0
+    x.reshape(n_tok, cols)[5, -1] = np.inf
+    x.reshape(n_tok, cols)[6, 40] = 3e38
+    x.reshape(n_tok, cols)[7, 5] = np.nan
+    y, ref = run(oracle, dtype, 50, cols, n_tok, x=x)
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(y), nan) and nan.reshape(n_tok, 50)[7].all()
+    assert np.array_equal(y[~nan].view(np.uint32), ref[~nan].view(np.uint32))
