@@ -356,278 +356,318 @@ __device__ __forceinline__ bool tok_block(const AttnArgs& a, int p0, int n_seq, 
     return true;
 }
 
+// How many 256-key blocks token t's span touches.
+__device__ __forceinline__ int tok_blocks(const AttnArgs& a, int p0, int n_seq, int t) {
+    int first, last;
+    attn_span(a.window, p0 + t, n_seq, first, last);
+    return last / ATTN_BLOCK - first / ATTN_BLOCK + 1;
+}
+
 // The partials (scalar.rs:444-519, gemma3.cpp attn_block) of tokens
 // x * tq .. + tq - 1, heads of KV head y, over 256-key block z: rows
 // r = s * G + h (token slot s, head h), at most AT_NQ. Every row's values
 // are the CPU's: its scores, first maximum, weights, weight sum and V sum
-// over the token's own keys of the block, in key order. The workgroup stages
-// the block's K rows (then V rows) AT_KC at a time in LDS for all its rows.
-// Scores: thread (key j, half) holds K row j in registers and runs the
-// 8-lane FMA chains of its half's rows, the queries (the same for the whole
-// wave) read by scalar loads. V sums: thread (columns, row group) keeps the
-// chains o[r][i] of its rows and columns across the chunks. The LDS moves
-// about 4 bytes per FMA lane when the wave-uniform operand comes from LDS
-// (a broadcast read still returns 64 lanes' data), half the VALU's rate:
-// hence scalar queries, and several columns per weight read.
-constexpr int AT_KC = 128;  // keys per LDS chunk
+// over the token's own keys of the block, in key order.
+//
+// The scores and the V sums run on the f32 matrix unit: an output of
+// v_mfma_f32_16x16x4_f32 is four fused multiply-adds in k order, each rounded
+// once, so a score's 8-lane FMA chains are 8 matrix products over the head's
+// 8-chunks (added as hsum8 does, in registers) and a V sum's chain is one over
+// the keys. Operands come straight from global memory in the matrix layout:
+//   scores: lane (c, k) reads 16 bytes of K row c at 8-chunk 4 i + k (and as
+//           many values of query row c), the 8 chains' operands at once;
+//   V sums: lane (c, k) reads its columns HD / 16 * c .. of V row 4 i + k, one
+//           per 16-column tile (tile d is columns HD / 16 * c + d).
+// Waves take every fourth 16-key tile of the scores, then their column tiles
+// of the V sums for all rows, so that a converted operand serves both 16-row
+// tiles. Keys that only some rows have (a causal or window edge: a few) run
+// one per matrix instruction, the other k slots 0 * -0 (which leaves an
+// accumulator as it is), and only the rows that have the key take the result.
+//
+// The softmax keeps a row's scores in the registers of 8 lanes between one read
+// and one write of LDS. Three workgroups share a CU (two at head_dim 256), which
+// hides most of each one's loads and barriers: 184 registers, two workgroups,
+// measured 70 us where 166 and three take 51.
+//
+// Bound: latency and the imbalance of causal tiles above the f32 matrix rate
+// (14 us of matrix instructions; 4 of a tile's 32 rows are idle with 7 heads per KV
+// head). Qwen2.5-7B shape (28 / 4 heads of 128), 512
+// tokens: 51 us per layer, 123 with the FMAs on the vector unit fed from LDS
+// (4 bytes of LDS return per FMA); with tokens of one block finished here, the
+// merge after it 15 -> 12.
 constexpr int AT_NQ = 32;   // rows per workgroup at most (16 at head_dim 256: registers)
+constexpr int AT_CUS = 256;  // CUs of the GPU (workgroup order only)
+constexpr int AT_SC = ATTN_BLOCK + 4;  // floats per LDS row: rows 4 apart fall on other banks
 __host__ __device__ constexpr int at_nq(int hd) { return hd >= 256 ? 16 : AT_NQ; }
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 template <int HD>
-__global__ __launch_bounds__(256) void attn_tile_kernel(AttnArgs a) {
-    constexpr int KS = HD + 8;
-    static_assert(HD % 8 == 0 && 256 % HD == 0 && HD >= 32, "head_dim 32, 64, 128 or 256");
+__global__ __launch_bounds__(256, HD <= 128 ? 3 : 2) void attn_tile_kernel(AttnArgs a) {
+    static_assert(HD == 32 || HD == 64 || HD == 128 || HD == 256, "head_dim 32, 64, 128 or 256");
+    constexpr int NR = at_nq(HD) / 16;  // 16-row tiles
+    constexpr int KI = HD / 32;         // matrix instructions per chain
     extern __shared__ __align__(16) float lds[];
     __shared__ int tk0[AT_NQ], tk1[AT_NQ], tbi[AT_NQ], rk0[AT_NQ], rk1[AT_NQ];
+    __shared__ float linv[AT_NQ];  // 1 / weight sum of a row whose token has one block
     const int kvh = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int G = a.G, TQ = a.tq, NQ = TQ * G, t0 = blockIdx.x * TQ, pw = HD + 2, KVD = a.KV * HD;
+    const int c16 = lane & 15, kq = lane >> 4;
+    // A causal prompt's later token tiles have more keys. Workgroups a round of
+    // CUs apart share a CU, so every other round takes the tiles in reverse.
+    const bool rev = (((b * a.KV + kvh) * (int)gridDim.x) / AT_CUS) & 1;
+    const int tile = rev ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x;
+    const int G = a.G, TQ = a.tq, NQ = TQ * G, t0 = tile * TQ, pw = HD + 2, KVD = a.KV * HD;
     // The tile's key range in the block (every thread computes it).
     int p0, n_seq;
     attn_pos(a, p0, n_seq);
     int K0 = 1 << 30, K1 = -1;
+    int kf0 = 0, kf1 = 1 << 30;  // the keys that every token with any has
     for (int s = 0; s < TQ; ++s) {
         int k0, k1, bi;
         const bool on = tok_block(a, p0, n_seq, t0 + s, b, k0, k1, bi);
         if (tid == 0) {
             tk0[s] = on ? k0 : 1;
             tk1[s] = on ? k1 : 0;
-            tbi[s] = bi;
+            tbi[s] = on && tok_blocks(a, p0, n_seq, t0 + s) == 1 ? -1 : bi;
         }
         if (on) {
             K0 = k0 < K0 ? k0 : K0;
             K1 = k1 > K1 ? k1 : K1;
+            kf0 = k0 > kf0 ? k0 : kf0;
+            kf1 = k1 < kf1 ? k1 : kf1;
         }
     }
     if (K1 < 0) return;
     __syncthreads();
-    if (tid < NQ) {  // each row's key range: its token's
-        rk0[tid] = tk0[tid / G];
-        rk1[tid] = tk1[tid / G];
+    if (tid < AT_NQ) {  // each row's key range: its token's (none past NQ)
+        rk0[tid] = tid < NQ ? tk0[tid / G] : 1;
+        rk1[tid] = tid < NQ ? tk1[tid / G] : 0;
     }
-    float* sc = lds;                              // [NQ][256], key k at k - K0
-    float* mh = sc + NQ * ATTN_BLOCK;             // [AT_NQ]
-    uint16_t* kv = (uint16_t*)(mh + AT_NQ);       // [AT_KC][KS]
-    __syncthreads();
-    // Scores, chunk by chunk.
-    constexpr int PR = HD / 8;  // 16-byte pieces per row
-    for (int c0 = K0; c0 <= K1; c0 += AT_KC) {
-        const int nkc = K1 + 1 - c0 < AT_KC ? K1 + 1 - c0 : AT_KC;
-        for (int i = tid; i < nkc * PR; i += 256) {
-            const int j = i / PR, c = i - j * PR;
-            *(uint4*)(kv + j * KS + 8 * c) = *(const uint4*)(a.kc + (size_t)(c0 + j) * KVD + kvh * HD + 8 * c);
-        }
-        __syncthreads();
-        const int j = tid & (AT_KC - 1), half = tid >> 7;
-        if (j < nkc) {
-            const int key = c0 + j;
-            // The key's row in registers as f32 up to head_dim 128 (converted
-            // once for all rows); at 256 it is read from LDS with the queries.
-            constexpr bool F32ROW = HD <= 128;
-            const uint16_t* krow = kv + j * KS;
-            float kf[F32ROW ? HD : 1];
-            if (F32ROW) {
+    float* sc = lds;  // [at_nq][AT_SC], key k at k - K0
+    // The wave's share of the V sums: its column tiles for all rows (head_dim 32
+    // has two: there waves 2 and 3 take the second row tile instead). Its first
+    // V rows are asked for before the scores, those of the edge before the
+    // whole groups.
+    constexpr int CW = HD / 16;                  // columns per lane
+    constexpr int DT = HD >= 64 ? HD / 64 : 1;   // column tiles per wave
+    constexpr int RT = HD >= 64 ? NR : 1;        // row tiles per wave
+    const int d0 = HD >= 64 ? wave * DT : wave & 1, rt0 = HD >= 64 ? 0 : wave >> 1;
+    const int f1 = kf1 >= kf0 ? kf0 + ((kf1 + 1 - kf0) & ~3) : kf0;  // whole groups of 4: [kf0, f1)
+    const uint16_t* vb = a.vc + kvh * HD + CW * c16 + d0;
+    // This lane's DT values of V row `key`.
+    struct VRaw {
+        uint32_t w[DT >= 2 ? DT / 2 : 1];
+    };
+    const auto vload = [&](int key) {
+        VRaw v;
+        const uint16_t* p = vb + (size_t)key * KVD;
+        if (DT == 1)
+            v.w[0] = *p;
+        else if (DT == 2)
+            v.w[0] = *(const uint32_t*)p;
+        else
+            *(uint2*)v.w = *(const uint2*)p;
+        return v;
+    };
+    const auto vval = [&](const VRaw& v, int d) {
+        return __uint_as_float(d & 1 ? v.w[d >> 1] & 0xffff0000u : v.w[d >> 1] << 16);
+    };
+    constexpr int VB = 8, VM = 4;  // whole groups and edge keys loaded together
+    VRaw vr[2][VB], ve[VM];
+    const auto vfetch = [&](int g, VRaw(&x)[VB]) {  // past the last group: it again, unused
 #pragma unroll
-                for (int c = 0; c < PR; ++c) {
-                    const uint4 k8 = *(const uint4*)(krow + 8 * c);
-                    const uint32_t kw[4] = {k8.x, k8.y, k8.z, k8.w};
-#pragma unroll
-                    for (int l = 0; l < 8; ++l)
-                        kf[F32ROW ? 8 * c + l : 0] = bf16f((kw[l >> 1] >> (16 * (l & 1))) & 0xffffu);
-                }
-            }
-            // The two halves take token slots (or, with one token per tile,
-            // alternate heads). A row's queries are the same for the whole
-            // wave: read from global memory at a wave-uniform address (scalar
-            // loads; nothing in this kernel writes them), so the FMAs take
-            // them as scalar operands and only the K rows come from LDS.
-            const int hs = (TQ + 1) / 2;
-            const int ts0 = TQ >= 2 ? half * hs : 0, ts1 = TQ >= 2 ? (half + 1) * hs < TQ ? (half + 1) * hs : TQ : 1;
-            const int h0 = TQ >= 2 ? 0 : half, hstep = TQ >= 2 ? 1 : 2;
-            for (int ts = ts0; ts < ts1; ++ts) {
-                if (key < tk0[ts] || key > tk1[ts]) continue;
-                for (int h = h0; h < G; h += hstep) {
-                    const int r = ts * G + h;
-                    const float* __restrict__ qg =
-                        a.qkv + (size_t)__builtin_amdgcn_readfirstlane((t0 + ts) * a.QKV + (kvh * G + h) * HD);
-                    float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                    for (int c = 0; c < PR; ++c) {
-                        float qv[8];
-#pragma unroll
-                        for (int l = 0; l < 8; ++l) qv[l] = qg[8 * c + l];
-                        if (F32ROW) {
-#pragma unroll
-                            for (int l = 0; l < 8; ++l) acc[l] = __fmaf_rn(qv[l], kf[F32ROW ? 8 * c + l : 0], acc[l]);
-                        } else {
-                            const uint4 k8 = *(const uint4*)(krow + 8 * c);
-                            const uint32_t kw[4] = {k8.x, k8.y, k8.z, k8.w};
-#pragma unroll
-                            for (int l = 0; l < 8; ++l)
-                                acc[l] = __fmaf_rn(qv[l], bf16f((kw[l >> 1] >> (16 * (l & 1))) & 0xffffu), acc[l]);
-                        }
-                    }
-                    sc[r * ATTN_BLOCK + key - K0] = __fmul_rn(hsum8(acc), a.scale);
-                }
-            }
-        }
-        __syncthreads();
-    }
-    // Each row's maximum as `if m < v { m = v }` from its first key finds it:
-    // the first largest, NaN never taken unless the first score is NaN.
-    // Lane l scans keys 4l .. 4l + 3 of the row from -inf, then the lanes'
-    // results combine in key order.
-    for (int r = wave; r < NQ; r += 4) {
-        const int n = rk1[r] + 1 - rk0[r];
-        if (n <= 0) continue;
-        const float* sr = sc + r * ATTN_BLOCK + (rk0[r] - K0);
-        float m = -INFINITY;
-        for (int j = 4 * lane; j < 4 * lane + 4 && j < n; ++j)
-            if (m < sr[j]) m = sr[j];
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const float other = __shfl_xor(m, o, 64);
-            const float lo = (lane & o) ? other : m, hi = (lane & o) ? m : other;
-            m = lo < hi ? hi : lo;
-        }
-        if (lane == 0) mh[r] = sr[0] != sr[0] ? sr[0] : m;
-    }
-    __syncthreads();
-    for (int i = tid; i < NQ * ATTN_BLOCK; i += 256) {
-        const int r = i >> 8, k = K0 + (i & (ATTN_BLOCK - 1));
-        if (k >= rk0[r] && k <= rk1[r]) sc[i] = exp_lane(__fsub_rn(sc[i], mh[r]));
-    }
-    __syncthreads();
-    // The weight sums: lane l of row r's group of 8 adds weights l, l + 8, ..
-    // of the row's whole 8-chunks, hsum8, then the tail in order.
-    {
-        const int r = tid >> 3, l = tid & 7, s = r / G;
-        const int n = r < NQ ? rk1[r] + 1 - rk0[r] : 0, body = n & ~7;
-        const float* sr = sc + r * ATTN_BLOCK + (r < NQ ? rk0[r] - K0 : 0);
-        float vs = 0.0f;
-        for (int j = l; j < body; j += 8) vs = __fadd_rn(vs, sr[j]);
-        float ls = hsum8_lanes(vs);
-        if (n > 0 && l == 0) {
-            for (int j = body; j < n; ++j) ls = __fadd_rn(ls, sr[j]);
-            const int h = r - s * G;
-            float* part = a.parts + ((((size_t)(t0 + s) * a.KV + kvh) * a.nblk) + tbi[s]) * G * pw + h * pw;
-            part[HD] = mh[r];
-            part[HD + 1] = ls;
-        }
-    }
-    // V sums, chunk by chunk: the first key of a row writes w * v, the rest
-    // FMA. Each chain starts at -0, so the first key's FMA is exactly w * v
-    // (x + -0 = x for every x, signed zeros included). Thread (row group,
-    // column group) runs the chains of CPT adjacent columns of its rows, so
-    // each weight read (the same for the whole wave: one row group per wave
-    // from head_dim 64) feeds CPT FMAs. Keys every active row of the tile has
-    // ([kf0, kf1]) run without masks, four per step, the next step's reads
-    // issued before this step's FMAs; keys only some rows have run masked.
-    constexpr int CPT = HD >= 64 ? HD / 64 : 1, CG = HD / CPT, RG = 256 / CG;
-    constexpr int RPT = (at_nq(HD) + RG - 1) / RG;
-    const int cg = tid % CG, rg = tid / CG, ie = cg * CPT;
-    float o[RPT][CPT];
-#pragma unroll
-    for (int k = 0; k < RPT; ++k)
-#pragma unroll
-        for (int c = 0; c < CPT; ++c) o[k][c] = -0.0f;
-    int kf0 = K0, kf1 = K1;
-    for (int r = 0; r < NQ; ++r)
-        if (rk1[r] >= rk0[r]) {
-            kf0 = rk0[r] > kf0 ? rk0[r] : kf0;
-            kf1 = rk1[r] < kf1 ? rk1[r] : kf1;
-        }
-    const float* wrow[RPT];  // each row's weights, indexed by key (rows past NQ read row NQ - 1)
-#pragma unroll
-    for (int k = 0; k < RPT; ++k) wrow[k] = sc + (rg + RG * k < NQ ? rg + RG * k : NQ - 1) * ATTN_BLOCK - K0;
-    // CPT BF16 values of one V row at the thread's columns.
-    auto vload = [&](int j, float* v) {
-        const uint16_t* p = kv + j * KS + ie;
-        if (CPT == 1) {
-            v[0] = bf16f(p[0]);
-        } else if (CPT == 2) {
-            const uint32_t u = *(const uint32_t*)p;
-            v[0] = bf16f(u & 0xffffu);
-            v[CPT > 1 ? 1 : 0] = bf16f(u >> 16);
-        } else {
-            const uint2 u = *(const uint2*)p;
-            v[0] = bf16f(u.x & 0xffffu);
-            v[CPT > 1 ? 1 : 0] = bf16f(u.x >> 16);
-            v[CPT > 2 ? 2 : 0] = bf16f(u.y & 0xffffu);
-            v[CPT > 3 ? 3 : 0] = bf16f(u.y >> 16);
+        for (int u = 0; u < VB; ++u) {
+            const int k0 = kf0 + 4 * (g + u);
+            x[u] = vload((k0 < f1 ? k0 : f1 - 4) + kq);
         }
     };
-    for (int c0 = K0; c0 <= K1; c0 += AT_KC) {
-        const int nkc = K1 + 1 - c0 < AT_KC ? K1 + 1 - c0 : AT_KC, c1 = c0 + nkc;
-        __syncthreads();  // the previous chunk's (or the scores') reads are done
-        for (int i = tid; i < nkc * PR; i += 256) {
-            const int j = i / PR, c = i - j * PR;
-            *(uint4*)(kv + j * KS + 8 * c) = *(const uint4*)(a.vc + (size_t)(c0 + j) * KVD + kvh * HD + 8 * c);
+    const auto efetch = [&](int key) {
+#pragma unroll
+        for (int u = 0; u < VM; ++u) ve[u] = vload(key + u < K1 ? key + u : K1);
+    };
+    const int ng = (f1 - kf0) / 4;
+    if (ng > 0) vfetch(0, vr[0]);
+    // Scores.
+    {
+        f32x4 q[NR][KI][2];
+#pragma unroll
+        for (int rt = 0; rt < NR; ++rt) {
+            // Rows past NQ (and tokens past the batch) read the last row; their scores are never used.
+            const int r = 16 * rt + c16 < NQ ? 16 * rt + c16 : NQ - 1, s = r / G, h = r - s * G;
+            const int t = t0 + s < a.n_tok ? t0 + s : a.n_tok - 1;
+            const float* qr = a.qkv + (size_t)t * a.QKV + (kvh * G + h) * HD + 8 * kq;
+#pragma unroll
+            for (int i = 0; i < KI; ++i)
+#pragma unroll
+                for (int e = 0; e < 2; ++e) q[rt][i][e] = *(const f32x4*)(qr + 32 * i + 4 * e);
         }
-        __syncthreads();
-        // The unmasked keys of this chunk, from a multiple of 4 past K0.
-        int f0 = kf0 > c0 ? kf0 : c0, f1 = kf1 + 1 < c1 ? kf1 + 1 : c1;
-        f0 = K0 + ((f0 - K0 + 3) & ~3);
-        if (f1 < f0) f1 = f0;
-        f1 = f0 + ((f1 - f0) & ~3);
-        auto masked = [&](int key) {
-            float v[CPT];
-            vload(key - c0, v);
+        const uint16_t* kb = a.kc + kvh * HD + 8 * kq;
+        const int ntile = (K1 - K0) / 16 + 1;
+        uint4 kr[KI];
+        const auto fetch = [&](int kt) {  // keys past K1 reread it
+            const int key = K0 + 16 * kt + c16 < K1 ? K0 + 16 * kt + c16 : K1;
 #pragma unroll
-            for (int k = 0; k < RPT; ++k) {
-                const int r = rg + RG * k < NQ ? rg + RG * k : NQ - 1;
-                const bool on = rg + RG * k < NQ && key >= rk0[r] && key <= rk1[r];
-                const float w = wrow[k][key];
-#pragma unroll
-                for (int c = 0; c < CPT; ++c) {
-                    const float nv = __fmaf_rn(w, v[c], o[k][c]);
-                    o[k][c] = on ? nv : o[k][c];
-                }
-            }
+            for (int i = 0; i < KI; ++i) kr[i] = *(const uint4*)(kb + (size_t)key * KVD + 32 * i);
         };
-        for (int key = c0; key < f0 && key < c1; ++key) masked(key);
-        if (f0 < f1) {
-            // Two register sets used in turn (no copies): a step's FMAs run
-            // on one while the next step's reads fill the other.
-            float4 wa[RPT], wb[RPT];
-            float va[4][CPT], vb[4][CPT];
-            auto fetch = [&](int key, float4* w, float (*v)[CPT]) {
+        if (wave < ntile) fetch(wave);
+        for (int kt = wave; kt < ntile; kt += 4) {
+            float kf[KI][8];
 #pragma unroll
-                for (int k = 0; k < RPT; ++k) w[k] = *(const float4*)(wrow[k] + key);
+            for (int i = 0; i < KI; ++i) {
+                const uint32_t kw[4] = {kr[i].x, kr[i].y, kr[i].z, kr[i].w};
 #pragma unroll
-                for (int u = 0; u < 4; ++u) vload(key - c0 + u, v[u]);
-            };
-            auto step = [&](const float4* w, const float (*v)[CPT]) {
-#pragma unroll
-                for (int k = 0; k < RPT; ++k) {
-                    const float w4[4] = {w[k].x, w[k].y, w[k].z, w[k].w};
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-#pragma unroll
-                        for (int c = 0; c < CPT; ++c) o[k][c] = __fmaf_rn(w4[u], v[u][c], o[k][c]);
-                }
-            };
-            fetch(f0, wa, va);
-            int key = f0;
-            for (; key + 8 <= f1; key += 8) {
-                fetch(key + 4, wb, vb);
-                step(wa, va);
-                if (key + 8 < f1) fetch(key + 8, wa, va);
-                step(wb, vb);
+                for (int l = 0; l < 8; ++l)
+                    kf[i][l] = __uint_as_float(l & 1 ? kw[l >> 1] & 0xffff0000u : kw[l >> 1] << 16);
             }
-            if (key < f1) step(wa, va);
+            if (kt + 4 < ntile) fetch(kt + 4);
+#pragma unroll
+            for (int rt = 0; rt < NR; ++rt) {
+                f32x4 acc[8];
+#pragma unroll
+                for (int l = 0; l < 8; ++l) acc[l] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int i = 0; i < KI; ++i)
+#pragma unroll
+                    for (int l = 0; l < 8; ++l)
+                        acc[l] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[rt][i][l >> 2][l & 3], kf[i][l], acc[l], 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float v[8];
+#pragma unroll
+                    for (int l = 0; l < 8; ++l) v[l] = acc[l][e];
+                    sc[(16 * rt + 4 * kq + e) * AT_SC + 16 * kt + c16] = __fmul_rn(hsum8(v), a.scale);
+                }
+            }
         }
-        for (int key = f1 > f0 ? f1 : f0; key < c1; ++key)
-            if (key >= c0) masked(key);
     }
+    __syncthreads();
+    // The weights, their sum and the row's maximum: lanes l = 0 .. 7 of a row
+    // hold its keys l, l + 8, .. in registers. The maximum is the first key's
+    // score if that is NaN, else the largest (a NaN later is never taken); which
+    // of two equal zeros it is changes nothing computed from it. The sum is the
+    // reference's: lane l adds its weights of whole 8-chunks in key order,
+    // hsum8, then the tail in order.
+    {
+        const int r = tid >> 3, l = tid & 7;
+        const int n = r < NQ ? rk1[r] + 1 - rk0[r] : 0, body = n >> 3;
+        float* sr = sc + (n > 0 ? r * AT_SC + rk0[r] - K0 : 0);
+        const int steps = (K1 - K0) / 8 + 1;  // of the tile's longest row
+        float v[ATTN_BLOCK / 8];
+        float m = -INFINITY;
 #pragma unroll
-    for (int k = 0; k < RPT; ++k) {
-        const int r = rg + RG * k;
-        if (r >= NQ || rk1[r] < rk0[r]) continue;
-        const int s = r / G, h = r - s * G;
-        float* dst = a.parts + ((((size_t)(t0 + s) * a.KV + kvh) * a.nblk) + tbi[s]) * G * pw + h * pw + ie;
+        for (int i = 0; i < ATTN_BLOCK / 8; ++i) {
+            if (i >= steps) break;
+            v[i] = l + 8 * i < n ? sr[l + 8 * i] : -INFINITY;
+            m = fmaxf(m, v[i]);
+        }
+        m = fmaxf(m, dpp_f<0xB1>(m));
+        m = fmaxf(m, dpp_f<0x4E>(m));
+        m = fmaxf(m, dpp_f<0x141>(m));
+        const float first = __shfl(v[0], lane & 56, 64);
+        if (first != first) m = first;
+        float vs = 0.0f, tail = 0.0f;
 #pragma unroll
-        for (int c = 0; c < CPT; ++c) dst[c] = o[k][c];
+        for (int i = 0; i < ATTN_BLOCK / 8; ++i) {
+            if (i >= steps) break;
+            const float w = exp_lane(__fsub_rn(v[i], m));
+            if (l + 8 * i < n) sr[l + 8 * i] = w;
+            if (i < body) vs = __fadd_rn(vs, w);
+            if (i == body) tail = w;
+        }
+        float ls = hsum8_lanes(vs);
+#pragma unroll
+        for (int j = 0; j < 7; ++j) {
+            const float t = __shfl(tail, (lane & 56) + j, 64);
+            if (8 * body + j < n) ls = __fadd_rn(ls, t);
+        }
+        if (n > 0 && l == 0) {
+            const int s = r / G, h = r - s * G;
+            if (tbi[s] < 0) {
+                linv[r] = ls > 0.0f ? __fdiv_rn(1.0f, ls) : 0.0f;
+            } else {
+                float* part = a.parts + ((((size_t)(t0 + s) * a.KV + kvh) * a.nblk) + tbi[s]) * G * pw + h * pw;
+                part[HD] = m;
+                part[HD + 1] = ls;
+            }
+        }
     }
+    __syncthreads();
+    // V sums. The first key of a row writes w * v, the rest FMA: each chain starts
+    // at -0, so the first FMA is exactly w * v (x + -0 = x for every x, signed
+    // zeros included).
+    f32x4 o[RT][DT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int d = 0; d < DT; ++d) o[rt][d] = f32x4{-0.0f, -0.0f, -0.0f, -0.0f};
+    const float* wr = sc + (16 * rt0 + c16) * AT_SC - K0;  // the weights of row c16 of the wave's first row tile
+    // Keys k .. last, one per matrix instruction; ve holds the first VM's V rows.
+    const auto edge = [&](int k, int last) {
+        for (; k <= last; k += VM) {
+#pragma unroll
+            for (int u = 0; u < VM; ++u) {
+                const int key = k + u;
+                if (key > last) break;
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    const float w = kq == 0 ? wr[16 * rt * AT_SC + key] : 0.0f;
+#pragma unroll
+                    for (int d = 0; d < DT; ++d) {
+                        const f32x4 n = __builtin_amdgcn_mfma_f32_16x16x4f32(w, kq == 0 ? vval(ve[u], d) : -0.0f,
+                                                                             o[rt][d], 0, 0, 0);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int r = 16 * (rt0 + rt) + 4 * kq + e;
+                            o[rt][d][e] = key >= rk0[r] && key <= rk1[r] ? n[e] : o[rt][d][e];
+                        }
+                    }
+                }
+            }
+            if (k + VM <= last) efetch(k + VM);
+        }
+    };
+    if (K0 < kf0) {
+        efetch(K0);
+        edge(K0, kf0 - 1 < K1 ? kf0 - 1 : K1);
+    }
+    const int e0 = f1 > K0 ? f1 : K0;  // the keys past the whole groups
+    efetch(e0);
+    const auto groups = [&](int g, const VRaw(&x)[VB]) {
+#pragma unroll
+        for (int u = 0; u < VB; ++u) {
+            const int k0 = kf0 + 4 * (g + u);
+            if (k0 >= f1) break;
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const float w = wr[16 * rt * AT_SC + k0 + kq];
+#pragma unroll
+                for (int d = 0; d < DT; ++d)
+                    o[rt][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, vval(x[u], d), o[rt][d], 0, 0, 0);
+            }
+        }
+    };
+    for (int g = 0; g < ng; g += 2 * VB) {
+        vfetch(g + VB, vr[1]);
+        groups(g, vr[0]);
+        vfetch(g + 2 * VB, vr[0]);
+        groups(g + VB, vr[1]);
+    }
+    edge(e0, K1);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int r = 16 * (rt0 + rt) + 4 * kq + e;
+            if (r >= NQ || rk1[r] < rk0[r]) continue;
+            const int s = r / G, h = r - s * G;
+            // The token's only block: finished as attn_merge_kernel does for one partial.
+            const bool one = tbi[s] < 0;
+            float* dst = one ? a.out + (size_t)(t0 + s) * (a.KV * G * HD) + (kvh * G + h) * HD + CW * c16 + d0
+                             : a.parts + ((((size_t)(t0 + s) * a.KV + kvh) * a.nblk) + tbi[s]) * G * pw + h * pw +
+                                   CW * c16 + d0;
+#pragma unroll
+            for (int d = 0; d < DT; ++d) dst[d] = one ? __fmul_rn(o[rt][d][e], linv[r]) : o[rt][d][e];
+        }
 }
 
 // Batch u0 .. u0 + U - 1 of a thread's 16-byte pieces of cache rows k0 ..
@@ -994,13 +1034,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 // (scalar.rs:521-537, with glibc's expf), then each head's o / l
 // (scalar.rs:539-548) into out[t][head * hd ..]; qo.q != NULL (one token):
 // the output also quantized into qo (head_dim a multiple of 32, so every
-// half-wave of an iteration holds one block).
+// half-wave of an iteration holds one block). Tokens of a longer batch whose
+// span is one block are finished by attn_tile_kernel already.
 __global__ __launch_bounds__(1024) void attn_merge_kernel(AttnArgs a, QOut qo) {
     const int t = blockIdx.y, kvh = blockIdx.x, hd = a.hd, G = a.G, pw = hd + 2, hd8 = hd & ~7;
     int p0, n_seq, first, last;
     attn_pos(a, p0, n_seq);
     attn_span(a.window, p0 + t, n_seq, first, last);
     const int nb = last / ATTN_BLOCK - first / ATTN_BLOCK + 1;
+    if (a.n_tok > 1 && nb == 1) return;
     const float* P = a.parts + ((size_t)t * a.KV + kvh) * a.nblk * G * pw;
     for (int idx = threadIdx.x; idx < G * hd; idx += blockDim.x) {
         const int h = idx / hd, i = idx - h * hd;
@@ -1212,8 +1254,7 @@ int nngl_create(const nng_config* cfg, const float* norms, const float* biases, 
         return 1;
     }
     m->tq = G >= at_nq(hd) ? 1 : at_nq(hd) / G;
-    const size_t nq = (size_t)m->tq * G;
-    m->lds_attn = nq * ATTN_BLOCK * 4 + AT_NQ * 4 + (size_t)AT_KC * (hd + 8) * 2;
+    m->lds_attn = (size_t)at_nq(hd) * AT_SC * 4;
     if (m->lds_attn > (size_t)LDS_MAX) {
         m->err = "the attention tile exceeds the LDS";
         return 1;
