@@ -171,13 +171,14 @@ ActLayout act_layout(size_t cols, size_t n_tok, int act = NNH_ACT_I8) {
     return l;
 }
 
-void launch_quantize(int act, const float* x, size_t x_stride, size_t cols, size_t n_tok, uint8_t* a,
+// `parts`: of an MX buffer, what to write (nnh::MxParts).
+void launch_quantize(int act, const float* x, size_t x_stride, size_t cols, size_t n_tok, uint8_t* a, int parts,
                      hipStream_t st) {
     const ActLayout l = act_layout(cols, n_tok, act);
     if (act == NNH_ACT_MXI8)
         nnh::launch_quantize_mx(x, x_stride, (int)cols, (int)n_tok, (int8_t*)a, (uint16_t*)(a + l.off_s),
                                 (double*)(a + l.off_sx), (float*)(a + l.off_sxT), nnh::gemm_tok_pad((int)n_tok),
-                                (uint16_t*)(a + l.off_xb), (uint16_t*)(a + l.off_xl), st);
+                                (uint16_t*)(a + l.off_xb), (uint16_t*)(a + l.off_xl), parts, st);
     else
         nnh::launch_quantize_act(x, x_stride, (int)cols, (int)n_tok, (int8_t*)a, (uint16_t*)(a + l.off_s),
                                  (double*)(a + l.off_sx), (float*)(a + l.off_sxT), nnh::gemm_tok_pad((int)n_tok), st);
@@ -246,7 +247,9 @@ int run_gemv(const nnh_weight* w, const float* x, size_t x_stride, float* y, siz
                  nnh::launch_gemv_i8_qx(w->dtype, w->qs, w->sc, w->sb, x, rows, nb, y, st))) {
         // (One vector at most rows: quantized in the GEMV's own prologue.)
         const ActLayout l = act_layout(w->cols, n_tok, act);
-        launch_quantize(act, x, x_stride, w->cols, n_tok, scratch, st);
+        // Only this call's matmul reads the buffer, so what it does not read stays unwritten.
+        launch_quantize(act, x, x_stride, w->cols, n_tok, scratch,
+                        n_tok >= GEMM_MIN_TOKENS ? nnh::MX_PART_GEMM : nnh::MX_PART_INT8, st);
         launch_i8(w, act, scratch, n_tok, y, y_stride, scratch + l.bytes, st);
     }
     NNH_HIP(hipGetLastError());
@@ -870,7 +873,8 @@ int nnh_quantize_act_ex_dev(int act, const float* x, size_t x_stride, size_t col
     if (n_tok == 0) return NNH_OK;
     if (!x || !buf) return fail(NNH_E_INVALID, "quantize: null pointer");
     if (cols >= ((size_t)1 << 31) || n_tok * cols >= ((size_t)1 << 30)) return fail(NNH_E_INVALID, "quantize: too large");
-    launch_quantize(act, x, n_tok > 1 ? x_stride : cols, cols, n_tok, (uint8_t*)buf, (hipStream_t)stream);
+    launch_quantize(act, x, n_tok > 1 ? x_stride : cols, cols, n_tok, (uint8_t*)buf,
+                    nnh::MX_PART_INT8 | nnh::MX_PART_GEMM, (hipStream_t)stream);
     NNH_HIP(hipGetLastError());
     return NNH_OK;
 }

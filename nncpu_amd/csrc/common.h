@@ -209,8 +209,11 @@ void launch_block_dots(int dtype, const uint8_t* qs, const int8_t* aq, int rows,
 // MX int8 path (kernels_mx.hip): power-of-two activation scales and the BF16
 // MFMA GEMM. nbp8 = nb rounded up to whole 8-block groups.
 int mx_nbp8(int nb);
+// parts: what is written, the int8 layout (q, s, sx, sxT: the kernels up to 16
+// vectors), the GEMM's operands (xb, xl), or both.
+enum MxParts { MX_PART_INT8 = 1, MX_PART_GEMM = 2 };
 void launch_quantize_mx(const float* x, size_t x_stride, int cols, int n_tok, int8_t* q, uint16_t* s, double* sx,
-                        float* sxT, int tok_pad, uint16_t* xb, uint16_t* xl, hipStream_t st);
+                        float* sxT, int tok_pad, uint16_t* xb, uint16_t* xl, int parts, hipStream_t st);
 size_t mx_bias_bytes(int rows, int nb);    // Q4 biases twice, rows padded
 int mx_xl_tok(int n_tok);                  // GEMM token tiles' worth of tokens
 size_t mx_xl_bytes(int n_tok, int nb);     // X limbs, tokens padded to mx_xl_tok

@@ -21,38 +21,58 @@ namespace {
 
 // ---- activation quantizer: quant.rs:31-60 on the device ----------------------
 
-// One 32-lane half-wave per block of 32 values.
+// Eight lanes per block of 32 values, four values a lane: the block's maximum
+// and quant sum are three DPP steps each (a lane per value took ten LDS-crossbar
+// exchanges and four times the scale arithmetic per value: VALU-bound, 10.8 us
+// at 512 vectors of 3584 in the kernel trace, 6.3 this way).
+//   TK = 8, K = 4: a wave takes 8 vectors x 4 consecutive blocks (every load and
+//     store a whole 128- or 32-byte run), its loads in flight together; from
+//     QUANT_TILE_MIN vectors.
+//   TK = 1, K = 1: a wave takes 8 consecutive blocks; few vectors (latency).
+constexpr int QUANT_TILE_MIN = 17;
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int TK, int K>
 __global__ __launch_bounds__(256) void quantize_act_kernel(const float* __restrict__ x, size_t x_stride, int cols,
                                                            int n_tok, int8_t* __restrict__ q,
                                                            uint16_t* __restrict__ s, double* __restrict__ sx,
                                                            float* __restrict__ sxT, int tok_pad) {
-    const int nb = cols >> 5;
-    const int k = threadIdx.x & 31;
-    const int blk = blockIdx.x * 8 + (threadIdx.x >> 5);
-    const bool valid = blk < nb * n_tok;
-    const int bb = valid ? blk : 0;
-    const int t = bb / nb, b = bb - t * nb;
-    float v = x[(size_t)t * x_stride + 32 * (size_t)b + k];
-    float a = q8_abs(v);
+    const int nb = cols >> 5, p = threadIdx.x & 7, grp = threadIdx.x >> 3;
+    int t, b0;
+    if (TK == 8) {
+        t = blockIdx.y * 8 + (grp & 7);
+        b0 = (blockIdx.x * 4 + (grp >> 3)) * K;
+    } else {
+        const int blk = blockIdx.x * 32 + grp;
+        t = blk / nb;
+        b0 = blk - t * nb;
+    }
+    const float* xr = x + (size_t)(t < n_tok ? t : n_tok - 1) * x_stride + 4 * p;  // loads stay in bounds; stores are skipped
+    f4u v[K];
 #pragma unroll
-    for (int m = 16; m >= 1; m >>= 1) a = fmaxf(a, __shfl_xor(a, m, 32));
-    const Q8Scale qs = q8_scale(a);
-    const uint32_t sbits = qs.bits;
-    const float scale = qs.scale;
-    const int qi = q8_quant(v, qs.inv);
-    int qsum = qi;
+    for (int k = 0; k < K; ++k) v[k] = *(const f4u*)(xr + 32 * (size_t)(b0 + k < nb ? b0 + k : nb - 1));
 #pragma unroll
-    for (int m = 16; m >= 1; m >>= 1) qsum += __shfl_xor(qsum, m, 32);
-    if (!valid) return;
-    q[(size_t)t * cols + 32 * (size_t)b + k] = (int8_t)qi;
-    if (k == 0) {
-        s[(size_t)t * nb + b] = (uint16_t)sbits;
-        sx[2 * ((size_t)t * nb + b)] = (double)scale;
-        sx[2 * ((size_t)t * nb + b) + 1] = (double)scale * (double)qsum;  // exact: s_x * sum(q_x)
-        // Block-major f32 copies for the GEMM: [b][tok_pad] scale, then [b][tok_pad] scale * sum(q).
-        if (sxT) {
-            sxT[(size_t)b * tok_pad + t] = scale;
-            sxT[(size_t)nb * tok_pad + (size_t)b * tok_pad + t] = scale * (float)qsum;  // exact: 8 + 13 bits
+    for (int k = 0; k < K; ++k) {
+        const float a = max8(fmaxf(fmaxf(q8_abs(v[k][0]), q8_abs(v[k][1])), fmaxf(q8_abs(v[k][2]), q8_abs(v[k][3]))));
+        const Q8Scale qs = q8_scale(a);
+        int qi[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) qi[e] = q8_quant(v[k][e], qs.inv);
+        const int qsum = sum8(qi[0] + qi[1] + qi[2] + qi[3]);
+        const int b = b0 + k;
+        if (b >= nb || t >= n_tok) continue;
+        *(uint32_t*)(q + (size_t)t * cols + 32 * (size_t)b + 4 * p) =
+            (uint32_t)(qi[0] & 255) | (uint32_t)(qi[1] & 255) << 8 | (uint32_t)(qi[2] & 255) << 16 |
+            (uint32_t)(qi[3] & 255) << 24;
+        if (p == 0) {
+            const size_t i = (size_t)t * nb + b;
+            s[i] = (uint16_t)qs.bits;
+            *(double2*)(sx + 2 * i) = double2{(double)qs.scale, (double)qs.scale * (double)qsum};  // exact: s_x * sum(q_x)
+            // Block-major f32 copies for the GEMM: [b][tok_pad] scale, then [b][tok_pad] scale * sum(q).
+            if (sxT) {
+                sxT[(size_t)b * tok_pad + t] = qs.scale;
+                sxT[(size_t)nb * tok_pad + (size_t)b * tok_pad + t] = qs.scale * (float)qsum;  // exact: 8 + 13 bits
+            }
         }
     }
 }
@@ -958,8 +978,13 @@ void launch_pack_sb(const uint16_t* sc, const uint16_t* bi, uint32_t* sb, size_t
 
 void launch_quantize_act(const float* x, size_t x_stride, int cols, int n_tok, int8_t* q, uint16_t* s, double* sx,
                          float* sxT, int tok_pad, hipStream_t st) {
-    int blocks = (cols / 32) * n_tok;
-    quantize_act_kernel<<<ceil_div(blocks, 8), 256, 0, st>>>(x, x_stride, cols, n_tok, q, s, sx, sxT, tok_pad);
+    const int nb = cols / 32;
+    if (n_tok >= QUANT_TILE_MIN)
+        quantize_act_kernel<8, 4><<<dim3(ceil_div(nb, 16), ceil_div(n_tok, 8)), 256, 0, st>>>(x, x_stride, cols, n_tok,
+                                                                                               q, s, sx, sxT, tok_pad);
+    else
+        quantize_act_kernel<1, 1><<<ceil_div((long)nb * n_tok, 32), 256, 0, st>>>(x, x_stride, cols, n_tok, q, s, sx,
+                                                                                   sxT, tok_pad);
 }
 
 void launch_gemv_i8(int dtype, const uint8_t* qs, const uint16_t* scales, const uint16_t* biases, const uint32_t* sb,

@@ -56,6 +56,7 @@
 // quarter (Q4) of a BF16 copy's, and no such copy is kept.
 
 #include "common.h"
+#include "q8_act.h"
 
 namespace nnh {
 namespace {
@@ -72,14 +73,6 @@ constexpr int MX_TM_Q = 256;       // tokens per GEMM tile (the quantizer's xb t
 constexpr int MX_MIN_UNITS = 2;    // groups per workgroup at least
 static_assert(MX_KS * MX_NS == MX_GRP, "whole stages per group");
 
-__device__ __forceinline__ int rint_sat_mx(float v) {
-    float r = __builtin_rintf(v);
-    if (!(r == r)) return 0;
-    if (r >= 2147483648.0f) return 2147483647;
-    if (r <= -2147483648.0f) return (int)0x80000000;
-    return (int)r;
-}
-
 // ---- quantizer ---------------------------------------------------------------
 
 // The exponent E of a block's power-of-two scale: the least E with
@@ -95,59 +88,73 @@ __device__ __forceinline__ int mx_exponent(float amax) {
     return e < -126 ? -126 : (e > 127 ? 127 : e);
 }
 
-// One 32-lane half-wave per block of 32 values; blocks past nb (up to the
-// group-padded nbp8) and tokens past n_tok (up to xl_tok, whole GEMM token
-// tiles) only write zeros: the limbs of xl, and for tokens past n_tok the
-// xb values.
+// Eight lanes per block of 32 values, four values a lane (max and sum: three DPP
+// steps each); a wave takes 8 tokens x 4 consecutive blocks, so its loads are
+// 128-byte runs in flight together and its BF16 stores whole runs of the tiled
+// layout (a half-wave per block, a value a lane: VALU-bound, 42 us at 512 tokens
+// of 18944 and 10.7 of 3584 in the kernel trace, 14.8 and 6.4 this way). Blocks past nb (up to the group-padded nbp8) and
+// tokens past n_tok (up to xl_tok, whole GEMM token tiles) only write zeros: the
+// limbs of xl, and for tokens past n_tok the xb values. PARTS: which parts of
+// the buffer are written (MxParts).
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+constexpr int MXQ_K = 4;  // blocks per thread
+
+template <int PARTS>
 __global__ __launch_bounds__(256) void quantize_mx_kernel(const float* __restrict__ x, size_t x_stride, int cols,
                                                           int n_tok, int nbp8, int8_t* __restrict__ q,
                                                           uint16_t* __restrict__ s, double* __restrict__ sx,
                                                           float* __restrict__ sxT, int tok_pad, int xl_tok,
                                                           uint16_t* __restrict__ xb, uint16_t* __restrict__ xl) {
-    const int nb = cols >> 5;
-    const int k = threadIdx.x & 31;
-    const int blk = blockIdx.x * 8 + (threadIdx.x >> 5);
-    if (blk >= nbp8 * xl_tok) return;  // uniform per half-wave
-    const int t = blk / nbp8, b = blk - t * nbp8;
+    constexpr bool INT8 = PARTS & MX_PART_INT8, GEMM = PARTS & MX_PART_GEMM;
+    const int nb = cols >> 5, p = threadIdx.x & 7, grp = threadIdx.x >> 3;
+    const int t = blockIdx.y * 8 + (grp & 7), b0 = (blockIdx.x * 4 + (grp >> 3)) * MXQ_K;  // xl_tok, nbp8: multiples of 8
+    const float* xr = x + (size_t)(t < n_tok ? t : n_tok - 1) * x_stride + 4 * p;  // loads stay in bounds
+    f4u v[MXQ_K];
+#pragma unroll
+    for (int k = 0; k < MXQ_K; ++k) v[k] = *(const f4u*)(xr + 32 * (size_t)(b0 + k < nb ? b0 + k : nb - 1));
     // xb tiled: [token tile][block][token in tile][32], 16-byte chunks of a
     // row swizzled as the GEMM's LDS rows are (chunk c at c ^ ((row >> 2) & 3)).
     const int tt = t / MX_TM_Q, tr = t % MX_TM_Q;
-    const size_t xe = (((size_t)tt * nb + b) * MX_TM_Q + tr) * 32 + (((k >> 3) ^ ((tr >> 2) & 3)) << 3) + (k & 7);
-    if (b >= nb || t >= n_tok) {
-        if (k < 2) xl[((size_t)t * nbp8 + b) * 2 + k] = 0;
-        if (b < nb) xb[xe] = 0;
-        return;
-    }
-    const float v = x[(size_t)t * x_stride + 32 * (size_t)b + k];
-    // amax over the block, NaN skipped (as nncpu's encoder's `v.abs() > amax`).
-    float a = fabsf(v);
-    a = (a == a) ? a : 0.0f;
+    uint16_t* xw = xb + ((size_t)tt * nb * MX_TM_Q + tr) * 32 + (((p >> 1) ^ ((tr >> 2) & 3)) << 3) + 4 * (p & 1);
 #pragma unroll
-    for (int m = 16; m >= 1; m >>= 1) a = fmaxf(a, __shfl_xor(a, m, 32));
-    const bool zero = !(a > 0.0f);
-    const int E = mx_exponent(a);
-    int qi = zero ? 0 : rint_sat_mx(__builtin_ldexpf(v, -E));  // v 2^-E: exact unless below 2^-126 (then |q| < 1)
-    qi = qi < -127 ? -127 : (qi > 127 ? 127 : qi);
-    int qsum = qi;
+    for (int k = 0; k < MXQ_K; ++k) {
+        // amax over the block, NaN skipped (as nncpu's encoder's `v.abs() > amax`).
+        const float a = max8(fmaxf(fmaxf(q8_abs(v[k][0]), q8_abs(v[k][1])), fmaxf(q8_abs(v[k][2]), q8_abs(v[k][3]))));
+        const bool zero = !(a > 0.0f);
+        const int E = mx_exponent(a);
+        const float scale = zero ? 0.0f : __uint_as_float((uint32_t)(E + 127) << 23);
+        int qi[4];
+        uint32_t w[4];
 #pragma unroll
-    for (int m = 16; m >= 1; m >>= 1) qsum += __shfl_xor(qsum, m, 32);
-    const float scale = zero ? 0.0f : __uint_as_float((uint32_t)(E + 127) << 23);
-    const size_t e = (size_t)t * cols + 32 * (size_t)b + k;
-    q[e] = (int8_t)qi;
-    // q 2^E as BF16: at most 7 significant bits, so the f32's low half is zero.
-    xb[xe] = (uint16_t)(__float_as_uint((float)qi * scale) >> 16);
-    if (k == 0) {
-        const float X = scale * (float)qsum;  // exact: <= 12 significant bits
-        s[(size_t)t * nb + b] = (uint16_t)(__float_as_uint(scale) >> 16);
-        sx[2 * ((size_t)t * nb + b)] = (double)scale;
-        sx[2 * ((size_t)t * nb + b) + 1] = (double)X;
-        sxT[(size_t)b * tok_pad + t] = scale;
-        sxT[(size_t)nb * tok_pad + (size_t)b * tok_pad + t] = X;
-        // X = hi + lo, hi its top 8 significant bits, lo the rest (<= 4 bits).
-        const uint32_t hb = __float_as_uint(X) & 0xFFFF0000u;
-        const float lo = X - __uint_as_float(hb);
-        xl[((size_t)t * nbp8 + b) * 2] = (uint16_t)(hb >> 16);
-        xl[((size_t)t * nbp8 + b) * 2 + 1] = (uint16_t)(__float_as_uint(lo) >> 16);
+        for (int e = 0; e < 4; ++e) {
+            const int r = zero ? 0 : rint_sat(__builtin_ldexpf(v[k][e], -E));  // v 2^-E: exact unless below 2^-126 (then |q| < 1)
+            qi[e] = r < -127 ? -127 : (r > 127 ? 127 : r);
+            w[e] = __float_as_uint((float)qi[e] * scale) >> 16;  // q 2^E as BF16: at most 7 significant bits
+        }
+        const int qsum = sum8(qi[0] + qi[1] + qi[2] + qi[3]);
+        const int b = b0 + k;
+        if (b >= nbp8 || t >= xl_tok) continue;
+        const bool in = b < nb && t < n_tok;
+        if (GEMM && b < nb)
+            *(uint2*)(xw + (size_t)b * MX_TM_Q * 32) = in ? make_uint2(w[0] | w[1] << 16, w[2] | w[3] << 16) : uint2{0, 0};
+        if (INT8 && in)
+            *(uint32_t*)(q + (size_t)t * cols + 32 * (size_t)b + 4 * p) =
+                (uint32_t)(qi[0] & 255) | (uint32_t)(qi[1] & 255) << 8 | (uint32_t)(qi[2] & 255) << 16 |
+                (uint32_t)(qi[3] & 255) << 24;
+        if (p == 0) {
+            const float X = scale * (float)qsum;  // exact: <= 12 significant bits
+            // X = hi + lo, hi its top 8 significant bits, lo the rest (<= 4 bits).
+            const uint32_t hb = __float_as_uint(X) & 0xFFFF0000u;
+            const float lo = X - __uint_as_float(hb);
+            if (GEMM) *(uint32_t*)(xl + ((size_t)t * nbp8 + b) * 2) = in ? (hb >> 16) | (__float_as_uint(lo) & 0xFFFF0000u) : 0u;
+            if (INT8 && in) {
+                const size_t i = (size_t)t * nb + b;
+                s[i] = (uint16_t)(__float_as_uint(scale) >> 16);
+                *(double2*)(sx + 2 * i) = double2{(double)scale, (double)X};
+                sxT[(size_t)b * tok_pad + t] = scale;
+                sxT[(size_t)nb * tok_pad + (size_t)b * tok_pad + t] = X;
+            }
+        }
     }
 }
 
@@ -728,11 +735,19 @@ int mx_nbp8(int nb) { return ceil_div(nb, MX_GRP) * MX_GRP; }
 int mx_xl_tok(int n_tok) { return ceil_div(n_tok, MX_TM) * MX_TM; }
 
 void launch_quantize_mx(const float* x, size_t x_stride, int cols, int n_tok, int8_t* q, uint16_t* s, double* sx,
-                        float* sxT, int tok_pad, uint16_t* xb, uint16_t* xl, hipStream_t st) {
+                        float* sxT, int tok_pad, uint16_t* xb, uint16_t* xl, int parts, hipStream_t st) {
     const int nbp8 = mx_nbp8(cols / 32), xl_tok = mx_xl_tok(n_tok);
-    const long blocks = (long)nbp8 * xl_tok;
-    quantize_mx_kernel<<<ceil_div(blocks, 8), 256, 0, st>>>(x, x_stride, cols, n_tok, nbp8, q, s, sx, sxT, tok_pad,
-                                                            xl_tok, xb, xl);
+    // Without the GEMM's parts no token past n_tok is touched.
+    const dim3 grid(ceil_div(nbp8, 4 * MXQ_K), parts == MX_PART_INT8 ? ceil_div(n_tok, 8) : xl_tok / 8);
+#define NNH_Q(P) \
+    quantize_mx_kernel<P><<<grid, 256, 0, st>>>(x, x_stride, cols, n_tok, nbp8, q, s, sx, sxT, tok_pad, xl_tok, xb, xl)
+    if (parts == MX_PART_INT8)
+        NNH_Q(MX_PART_INT8);
+    else if (parts == MX_PART_GEMM)
+        NNH_Q(MX_PART_GEMM);
+    else
+        NNH_Q(MX_PART_INT8 | MX_PART_GEMM);
+#undef NNH_Q
 }
 
 size_t mx_bias_bytes(int rows, int nb) { return (size_t)gemm_rows_pad(rows) * mx_nbp8(nb) * 4; }
