@@ -235,8 +235,10 @@ int run_gemv(const nnh_weight* w, const float* x, size_t x_stride, float* y, siz
              uint8_t* scratch, hipStream_t st) {
     const int rows = (int)w->rows, nb = (int)w->nb;
     if (w->dtype == NNH_BF16) {
-        nnh::launch_gemv_bf16(w->bpath, (const uint16_t*)w->raw, w->bl, rows, (int)w->cols, x, x_stride, (int)n_tok, y,
-                              y_stride, st);
+        if (!nnh::launch_gemm_bf16(w->bpath, (const uint16_t*)w->raw, rows, (int)w->cols, x, x_stride, (int)n_tok, y,
+                                   y_stride, st))
+            nnh::launch_gemv_bf16(w->bpath, (const uint16_t*)w->raw, w->bl, rows, (int)w->cols, x, x_stride, (int)n_tok,
+                                  y, y_stride, st);
     } else if (act == NNH_ACT_F32) {
         float* xsum = w->dtype == NNH_Q4S ? (float*)scratch : nullptr;
         if (!nnh::launch_gemm_f32(w->dtype, w->qs, w->fs, w->bi, x, x_stride, xsum, rows, nb, (int)w->nbp,

@@ -188,6 +188,11 @@ size_t bf16_layout_bytes(int path, size_t rows, size_t cols);  // 0 for the f64 
 void launch_relayout_bf16(int path, const uint16_t* raw, uint16_t* bl, int rows, int cols, hipStream_t st);
 void launch_gemv_bf16(int path, const uint16_t* raw, const uint16_t* bl, int rows, int cols, const float* x,
                       size_t x_stride, int n_tok, float* y, size_t y_stride, hipStream_t st);
+// The same for several vectors on the f32 matrix unit (kernels_f32_batch.hip);
+// raw: the weights as uploaded. False (nothing launched) on the f64 path, for
+// few vectors, or when x's rows are not 16-byte aligned.
+bool launch_gemm_bf16(int path, const uint16_t* raw, int rows, int cols, const float* x, size_t x_stride, int n_tok,
+                      float* y, size_t y_stride, hipStream_t st);
 void launch_encode_bf16(const float* w, size_t n, uint16_t* out, hipStream_t st);
 // GGUF tensor blocks -> f32 (kernels_gguf.hip): bytes and values per block
 // of a decodable ggml type; the decode itself (n a whole number of blocks).

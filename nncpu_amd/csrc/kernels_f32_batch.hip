@@ -49,6 +49,7 @@ struct BatchArgs {
     float* y;
     size_t xs, ys;
     int rows, nb, nbp, n_tok;
+    int rem;             // BF16: columns past the nb whole 32-blocks (a multiple of 8)
     int ttiles, tq, tr;  // token tiles; tile i holds tq (+ 1 for the first tr) groups of 16 vectors
     bool vec_y;          // y rows take 16-byte stores
 };
@@ -73,6 +74,19 @@ __device__ __forceinline__ void lds_barrier() {
 
 __device__ __forceinline__ f32x4 add4(f32x4 a, f32x4 b) {
     return f32x4{__fadd_rn(a[0], b[0]), __fadd_rn(a[1], b[1]), __fadd_rn(a[2], b[2]), __fadd_rn(a[3], b[3])};
+}
+
+// A lane's result tile column: rows row .. row + 3 of vector tok.
+__device__ __forceinline__ void store4(const BatchArgs& g, f32x4 r, int row, int tok) {
+    if (tok >= g.n_tok) return;
+    float* yp = g.y + (size_t)tok * g.ys + row;
+    if (g.vec_y && row + 4 <= g.rows) {
+        *(f32x4*)yp = r;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (row + e < g.rows) yp[e] = r[e];
+    }
 }
 
 template <int DT, int R, int NT, int H>
@@ -372,18 +386,22 @@ __device__ __forceinline__ void batch_body(const BatchArgs& g, unsigned char* ld
                 }
                 r = add4(r, b);
             }
-            if (tok < g.n_tok) {
-                float* yp = g.y + (size_t)tok * g.ys + row;
-                if (g.vec_y && row + 4 <= g.rows) {
-                    *(f32x4*)yp = r;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (row + e < g.rows) yp[e] = r[e];
-                }
-            }
+            store4(g, r, row, tok);
         }
     }
+}
+
+// A workgroup's row tile, first vector and 16-vector groups. Workgroups go
+// round-robin to the 8 XCDs; each XCD takes a contiguous range of logical ids,
+// the token tiles of a row tile side by side, so a row tile's weights are read
+// once into its L2.
+__device__ __forceinline__ void batch_tile(const BatchArgs& g, int& rt, int& tok0, int& nt) {
+    const int total = gridDim.x, per = total / 8, rem = total % 8, xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
+    const int id = xcd < rem ? xcd * (per + 1) + slot : rem * (per + 1) + (xcd - rem) * per + slot;
+    rt = id / g.ttiles;
+    const int tt = id - rt * g.ttiles;
+    nt = g.tq + (tt < g.tr ? 1 : 0);
+    tok0 = 16 * (tt * g.tq + min(tt, g.tr));
 }
 
 // NT: 16-vector groups of the largest token tile; a launch's tiles hold NT or
@@ -391,18 +409,246 @@ __device__ __forceinline__ void batch_body(const BatchArgs& g, unsigned char* ld
 template <int DT, int R, int NT, int H, int NS>
 __global__ __launch_bounds__(R * H * 256) void gemm_f32_kernel(BatchArgs g) {
     extern __shared__ __align__(16) unsigned char lds[];
-    // Workgroups go round-robin to the 8 XCDs; each XCD takes a contiguous
-    // range of logical ids, the token tiles of a row tile side by side, so a
-    // row tile's weights are read once into its L2.
-    const int total = gridDim.x, per = total / 8, rem = total % 8, xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
-    const int id = xcd < rem ? xcd * (per + 1) + slot : rem * (per + 1) + (xcd - rem) * per + slot;
-    const int rt = id / g.ttiles, tt = id - rt * g.ttiles;
-    const int nt = g.tq + (tt < g.tr ? 1 : 0);
-    const int tok0 = 16 * (tt * g.tq + min(tt, g.tr));
+    int rt, tok0, nt;
+    batch_tile(g, rt, tok0, nt);
     if (nt == NT)
         batch_body<DT, R, NT, H, NS>(g, lds, rt * 16 * R, tok0);
     else if constexpr (NT > 1)
         batch_body<DT, R, NT - 1, H, NS>(g, lds, rt * 16 * R, tok0);
+}
+
+// BF16 weights for several vectors, the same scheme (kernels_bf16.hip names the
+// reference's kernel per shape and its chains):
+//   ROW32       32 chains, element j of every 32-block: a wave's chains and the
+//               meeting as for Q8_0 above;
+//   QUAD, ROW8  8 chains over elements 8 i + l, i in order: a matrix instruction
+//               takes 4 values of i (32 columns), a wave the chain pair that is
+//               added first (QUAD l = 2 w, 2 w + 1, ROW8's hsum8 l = w, w + 4),
+//               so waves meet once, on (p0 + p1) + (p2 + p3).
+// A stage is 256 columns: 512 bytes per row of raw weights, in 16-byte pieces
+// XOR-swizzled by row. Measured (us; before: four vectors per pass of
+// gemv_bf16_kernel): 6144 x 1536, 16 vectors 38.6 -> 8.4, 6143 rows 38.8 -> 8.3;
+// 14336 x 4096 149 -> 34.4.
+template <int R, int NT>
+struct Bf16Lds {
+    static constexpr int X = NT * 16384;
+    static constexpr int STAGE = X + R * 8192;
+};
+
+template <int PATH, int R, int NT, int NS>
+__device__ __forceinline__ void bf16_body(const BatchArgs& g, unsigned char* lds, int row0, int tok0) {
+    using L = Bf16Lds<R, NT>;
+    constexpr bool WIDE = PATH == BF16_PATH_ROW32, QUAD = PATH == BF16_PATH_QUAD;
+    constexpr int NC = WIDE ? 8 : 2;           // chains per wave
+    constexpr int STEPS = WIDE ? 2 : 8;        // matrix instructions of a chain per stage
+    constexpr int NW = 4 * R, XC = 16 / NW;    // waves; x copies per wave, stage and vector group
+    constexpr int CP = NT * XC + 2;            // copies per wave and stage
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rg = wave >> 2, w = wave & 3, c16 = lane & 15, k = lane >> 4;
+    const int cols = 32 * g.nb + g.rem, nst = (cols + 255) / 256, full = cols / 256;
+    const uint32_t ring = (uint32_t)(uintptr_t)lds;
+
+    uint32_t xrow[NT];
+    const float* xb = g.x + (size_t)tok0 * g.xs;
+    const int v8 = 8 * (wave & 1) + (lane >> 3);
+    const uint32_t xc = 16 * ((lane & 7) ^ ((v8 >> 1) & 7));
+#pragma unroll
+    for (int t = 0; t < NT; ++t) xrow[t] = (uint32_t)min(16 * t + v8, g.n_tok - 1 - tok0) * (uint32_t)(g.xs * 4);
+    const int last = g.rows - 1 - row0;
+    const uint8_t* wb = g.qs + (size_t)row0 * cols * 2;
+    uint32_t wfull[2], wlast[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int r = 4 * w + 2 * i + (lane >> 5), c = (lane & 31) ^ r;  // row in the group, its piece
+        const uint32_t o = (uint32_t)min(16 * rg + r, last) * (uint32_t)(cols * 2);
+        wfull[i] = o + 16 * c;
+        wlast[i] = o + 16 * min(c, cols / 8 - 32 * (nst - 1) - 1);  // pieces past the row repeat its last one
+    }
+    const auto copy = [&](int i, int st, uint32_t buf) {
+        const uint32_t d = ring + buf;
+        if (i < NT * XC) {
+            const int t = i / XC, jj = i % XC, kk = (wave >> 1) + (NW / 2) * jj;
+            uint32_t o = xc + (uint32_t)(8 * st + kk) * 128;
+            if (st == nst - 1) o = min(o, (uint32_t)(cols * 4 - 16));
+            copy16(xb, xrow[t] + o, d + t * 16384 + (wave + NW * jj) * 1024);
+        } else {
+            const int j = i - NT * XC;
+            copy16(wb + (size_t)st * 512, st == nst - 1 ? wlast[j] : wfull[j],
+                   d + L::X + rg * 8192 + (2 * w + j) * 1024);
+        }
+    };
+#pragma unroll
+    for (int p = 0; p < NS - 1; ++p)
+#pragma unroll
+        for (int i = 0; i < CP; ++i) copy(i, min(p, nst - 1), p * L::STAGE);
+
+    f32x4 acc[NT][NC];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < NC; ++i) acc[t][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    const auto lo = [](uint32_t v) { return __uint_as_float(v << 16); };
+    const auto hi = [](uint32_t v) { return __uint_as_float(v & 0xffff0000u); };
+    // The weights' operands of step s: piece 4 s + k of the row (QUAD, ROW8), or
+    // the pieces of block 4 s + k.
+    const auto load_w = [&](uint32_t p, int s, float(&a)[NC]) {
+        const unsigned char* row = lds + p + L::X + rg * 8192 + c16 * 512;
+        if (WIDE) {
+            const int c = 4 * (4 * s + k) + (w >> 1);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint2 v = *(const uint2*)(row + 16 * ((c + 2 * h) ^ c16) + 8 * (w & 1));
+                a[4 * h % NC] = lo(v.x);
+                a[(4 * h + 1) % NC] = hi(v.x);
+                a[(4 * h + 2) % NC] = lo(v.y);
+                a[(4 * h + 3) % NC] = hi(v.y);
+            }
+        } else {
+            const unsigned char* q = row + 16 * ((4 * s + k) ^ c16);
+            if (QUAD) {
+                const uint32_t v = *(const uint32_t*)(q + 4 * w);
+                a[0] = lo(v);
+                a[1] = hi(v);
+            } else {
+                a[0] = lo(*(const uint16_t*)(q + 2 * w));
+                a[1] = lo(*(const uint16_t*)(q + 8 + 2 * w));
+            }
+        }
+    };
+    const int sw = (c16 >> 1) & 7;
+    const auto load_x = [&](uint32_t p, int s, int t, float(&b)[NC]) {
+        const unsigned char* x = lds + p + t * 16384 + (WIDE ? 4 * s + k : s) * 2048 + c16 * 128;
+        if (WIDE) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const f32x4 v = *(const f32x4*)(x + 16 * ((w + 4 * h) ^ sw));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) b[(4 * h + i) % NC] = v[i];
+            }
+        } else if (QUAD) {
+            const float2 v = *(const float2*)(x + 16 * ((2 * k + (w >> 1)) ^ sw) + 8 * (w & 1));
+            b[0] = v.x;
+            b[1] = v.y;
+        } else {
+            b[0] = *(const float*)(x + 16 * ((2 * k) ^ sw) + 4 * w);
+            b[1] = *(const float*)(x + 16 * ((2 * k + 1) ^ sw) + 4 * w);
+        }
+    };
+    uint32_t cur = 0, fill = (NS - 1) * L::STAGE;
+    const auto after = [&](uint32_t p) { return p == (NS - 1) * L::STAGE ? 0 : p + L::STAGE; };
+    constexpr int SLOTS = STEPS * NT * NC;
+    for (int st = 0; st < full; ++st) {
+        wait_vmcnt<CP*(NS - 2)>();
+        lds_barrier();
+        const int sf = min(st + NS - 1, nst - 1);
+        float a[2][NC], b[2][NC];
+        load_w(cur, 0, a[0]);
+        load_x(cur, 0, 0, b[0]);
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            if (s + 1 < STEPS) load_w(cur, s + 1, a[(s + 1) & 1]);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const int v = s * NT + t;
+                if (v + 1 < STEPS * NT) load_x(cur, (v + 1) / NT, (v + 1) % NT, b[(v + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < NC; ++i) {
+                    acc[t][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s & 1][i], b[v & 1][i], acc[t][i], 0, 0, 0);
+                    const int u = v * NC + i;
+#pragma unroll
+                    for (int e = u * CP / SLOTS; e < (u + 1) * CP / SLOTS; ++e) copy(e, sf, fill);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        fill = after(fill);
+        cur = after(cur);
+    }
+    if (full < nst) {  // the partial last stage: missing steps are 0 * -0
+        wait_vmcnt<0>();
+        lds_barrier();
+        const int left = WIDE ? (cols - 256 * full) / 32 : (cols - 256 * full) / 8;  // blocks / values of i
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            if (4 * s >= left) break;
+            const bool on = 4 * s + k < left;
+            float a[NC], b[NC];
+            load_w(cur, s, a);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                load_x(cur, s, t, b);
+#pragma unroll
+                for (int i = 0; i < NC; ++i)
+                    acc[t][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(on ? a[i] : 0.0f, on ? b[i] : -0.0f, acc[t][i], 0, 0,
+                                                                     0);
+            }
+        }
+    }
+
+    wait_vmcnt<0>();  // the repeated copies, before the ring is written over
+    lds_barrier();
+    if constexpr (WIDE) {
+        // As in batch_body: words 2 and 3 hand their chains to words 0 and 1.
+        unsigned char* m = lds + rg * 20 * 1024 + lane * 16;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            lds_barrier();
+            if (w >= 2)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) *(f32x4*)(m + ((w - 2) * 8 + i) * 1024) = acc[t][i % NC];
+            lds_barrier();
+            f32x4 v[4];
+            if (w < 2) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    v[i] = add4(add4(acc[t][i % NC], *(const f32x4*)(m + (w * 8 + i) * 1024)),
+                                add4(acc[t][(4 + i) % NC], *(const f32x4*)(m + (w * 8 + 4 + i) * 1024)));
+                    if (w == 1) *(f32x4*)(m + (16 + i) * 1024) = v[i];
+                }
+            }
+            lds_barrier();
+            if (w == 0) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = add4(v[i], *(const f32x4*)(m + (16 + i) * 1024));
+                store4(g, add4(add4(v[0], v[1]), add4(v[2], v[3])), row0 + 16 * rg + 4 * k, tok0 + 16 * t + c16);
+            }
+        }
+    } else {
+        unsigned char* m = lds + rg * 4 * NT * 1024 + lane * 16;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) *(f32x4*)(m + (4 * t + w) * 1024) = add4(acc[t][0], acc[t][1]);
+        lds_barrier();
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            if ((t & 3) != w) continue;
+            f32x4 p[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) p[i] = *(const f32x4*)(m + (4 * t + i) * 1024);
+            store4(g, add4(add4(p[0], p[1]), add4(p[2], p[3])), row0 + 16 * rg + 4 * k, tok0 + 16 * t + c16);
+        }
+    }
+}
+
+template <int PATH, int R, int NT, int NS>
+__global__ __launch_bounds__(R * 256) void gemm_bf16_kernel(BatchArgs g) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    int rt, tok0, nt;
+    batch_tile(g, rt, tok0, nt);
+    if (nt == NT)
+        bf16_body<PATH, R, NT, NS>(g, lds, rt * 16 * R, tok0);
+    else if constexpr (NT > 1)
+        bf16_body<PATH, R, NT - 1, NS>(g, lds, rt * 16 * R, tok0);
+}
+
+// The launch's token tiles: n16 groups of 16 vectors spread over tiles of at most nt.
+int token_tiles(BatchArgs& g, int nt) {
+    const int n16 = ceil_div(g.n_tok, 16);
+    g.ttiles = ceil_div(n16, nt);
+    g.tq = n16 / g.ttiles;
+    g.tr = n16 % g.ttiles;
+    return g.ttiles;
 }
 
 template <int DT, int R, int NT, int H, int NS>
@@ -415,29 +661,57 @@ void launch_batch(BatchArgs g, hipStream_t st) {
                                    hipFuncAttributeMaxDynamicSharedMemorySize, LDS) == hipSuccess;
     }();
     (void)once;
-    const int n16 = ceil_div(g.n_tok, 16);
-    g.ttiles = ceil_div(n16, NT);
-    g.tq = n16 / g.ttiles;
-    g.tr = n16 % g.ttiles;
-    gemm_f32_kernel<DT, R, NT, H, NS><<<ceil_div(g.rows, 16 * R) * g.ttiles, R * H * 256, LDS, st>>>(g);
+    const int tiles = token_tiles(g, NT);
+    gemm_f32_kernel<DT, R, NT, H, NS><<<ceil_div(g.rows, 16 * R) * tiles, R * H * 256, LDS, st>>>(g);
 }
 
-template <int DT>
-void launch_dt(const BatchArgs& g, hipStream_t st) {
+template <int PATH, int R, int NT, int NS>
+void launch_bf16(BatchArgs g, hipStream_t st) {
+    constexpr int LDS = NS * Bf16Lds<R, NT>::STAGE;
+    static_assert(LDS <= 160 * 1024 && LDS >= R * 20 * 1024, "the ring fits the LDS and holds the meeting area");
+    static const bool once = [] {
+        return hipFuncSetAttribute((const void*)gemm_bf16_kernel<PATH, R, NT, NS>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, LDS) == hipSuccess;
+    }();
+    (void)once;
+    const int tiles = token_tiles(g, NT);
+    gemm_bf16_kernel<PATH, R, NT, NS><<<ceil_div(g.rows, 16 * R) * tiles, R * 256, LDS, st>>>(g);
+}
+
+// The split with the least time: rounds of workgroups over the CUs times a
+// workgroup's time per stage of 256 columns (us, measured for Q8_0 at 14336 and
+// 4096 rows; BF16's is within a tenth): 0 one row group and 16 vectors per
+// workgroup, 1 the same with a workgroup or less per CU, 2 two row groups and
+// 32 vectors, 3 two and 64.
+int pick_split(const BatchArgs& g) {
     const int n16 = ceil_div(g.n_tok, 16), cus = cu_count();
-    // The split with the least time: rounds of workgroups over the CUs times a
-    // workgroup's time per stage (us, measured at 14336 and 4096 rows).
     const auto cost = [&](int r, int nt, double us) {
         const long wgs = (long)ceil_div(g.rows, 16 * r) * ceil_div(n16, nt);
         return (double)((wgs + cus - 1) / cus) * us;
     };
     const double c11 = cost(1, 1, 0.45), c22 = cost(2, 2, 1.42), c24 = cost(2, 4, 2.6);
-    const int pick = c24 <= c11 && c24 <= c22 ? 3 : c22 <= c11 ? 2 : (long)ceil_div(g.rows, 16) * n16 <= cus ? 0 : 1;
-    switch (pick) {
-        case 0: launch_batch<DT, 1, 1, 2, 3>(g, st); break;
-        case 1: launch_batch<DT, 1, 1, 1, 3>(g, st); break;
+    if (c24 <= c11 && c24 <= c22) return 3;
+    if (c22 <= c11) return 2;
+    return (long)ceil_div(g.rows, 16) * n16 <= cus ? 1 : 0;
+}
+
+template <int DT>
+void launch_dt(const BatchArgs& g, hipStream_t st) {
+    switch (pick_split(g)) {
+        case 1: launch_batch<DT, 1, 1, 2, 3>(g, st); break;
+        case 0: launch_batch<DT, 1, 1, 1, 3>(g, st); break;
         case 2: launch_batch<DT, 2, 2, 1, 3>(g, st); break;
         default: launch_batch<DT, 2, 4, 1, 2>(g, st); break;
+    }
+}
+
+template <int PATH>
+void launch_path(const BatchArgs& g, hipStream_t st) {
+    switch (pick_split(g)) {
+        case 0:
+        case 1: launch_bf16<PATH, 1, 1, 3>(g, st); break;
+        case 2: launch_bf16<PATH, 2, 2, 3>(g, st); break;
+        default: launch_bf16<PATH, 2, 4, 2>(g, st); break;
     }
 }
 
@@ -456,11 +730,29 @@ bool launch_gemm_f32(int dtype, const uint8_t* qs, const uint16_t* fs, const uin
     if (((uintptr_t)x & 15) || (x_stride & 3) || x_stride >= ((size_t)1 << 23) || nb >= (1 << 21)) return false;
     if (dtype == 2) launch_block_sums(x, x_stride, nb, n_tok, xsum, st);
     const BatchArgs g{qs, fs,       biases, x,  xsum, y, x_stride, y_stride,
-                      rows, nb, nbp, n_tok, 0, 0, 0, ((uintptr_t)y & 15) == 0 && (y_stride & 3) == 0};
+                      rows, nb, nbp, n_tok, 0, 0, 0, 0, ((uintptr_t)y & 15) == 0 && (y_stride & 3) == 0};
     if (dtype == 1)
         launch_dt<1>(g, st);
     else
         launch_dt<2>(g, st);
+    return true;
+}
+
+bool launch_gemm_bf16(int path, const uint16_t* raw, int rows, int cols, const float* x, size_t x_stride, int n_tok,
+                      float* y, size_t y_stride, hipStream_t st) {
+    // Few vectors stay on the chain kernel: measured, that against here, three
+    // vectors 6144 x 1536 8.0 / 8.3 us, 14336 x 4096 34.1 / 33.8, four 10.0 / 8.3.
+    if (path == BF16_PATH_F64 || n_tok < 4 || ((uintptr_t)x & 15) || (x_stride & 3) ||
+        x_stride >= ((size_t)1 << 23) || cols >= (1 << 26))
+        return false;
+    const BatchArgs g{(const uint8_t*)raw, nullptr, nullptr, x, nullptr, y, x_stride, y_stride, rows, cols / 32, 0, n_tok,
+                      cols % 32,           0,       0,       0, ((uintptr_t)y & 15) == 0 && (y_stride & 3) == 0};
+    if (path == BF16_PATH_QUAD)
+        launch_path<BF16_PATH_QUAD>(g, st);
+    else if (path == BF16_PATH_ROW8)
+        launch_path<BF16_PATH_ROW8>(g, st);
+    else
+        launch_path<BF16_PATH_ROW32>(g, st);
     return true;
 }
 

@@ -63,3 +63,26 @@ def test_f32_batch_special_values(oracle, dtype, cols):
     nan = np.isnan(ref)
     assert np.array_equal(np.isnan(y), nan) and nan.reshape(n_tok, 50)[7].all()
     assert np.array_equal(y[~nan].view(np.uint32), ref[~nan].view(np.uint32))
+
+
+# BF16: the 4-row kernel's chains (rows % 4 == 0), the 1-row kernel's 8 (cols % 32
+# != 0) and 32, around stages of 256 columns, 8- and 32-column steps.
+@pytest.mark.parametrize("rows,cols,n_tok,pad", [
+    (4, 8, 5, 0), (16, 264, 17, 4), (40, 520, 33, 0), (256, 1000, 64, 8), (4100, 512, 40, 0), (8208, 544, 16, 0),
+    (17, 24, 6, 0), (33, 248, 16, 4), (70, 1544, 65, 0), (1030, 264, 130, 0),
+    (1, 32, 4, 0), (31, 224, 18, 0), (257, 608, 49, 4), (4097, 288, 65, 0), (6, 320, 9, 3),
+])
+def test_bf16_batch_bit_exact(oracle, rows, cols, n_tok, pad):
+    rng = np.random.default_rng(rows * 7 + cols + n_tok)
+    w = oracle.f32_array_to_bf16(rng.standard_normal(rows * cols).astype(np.float32))
+    xs, ys = cols + pad, rows + pad
+    x = np.ldexp(rng.standard_normal(n_tok * xs), rng.integers(-30, 30, n_tok * xs)).astype(np.float32)
+    x[rng.integers(0, x.size, x.size // 8)] = -0.0
+    wt = N.Weight.bf16(w, rows, cols)
+    y = np.full(n_tok * ys, 7.0, np.float32)
+    N.gemv_batch(wt, x, xs, y, ys, n_tok)
+    want = oracle.gemv_bf16(w, x, rows, cols, n_tok, xs, ys)
+    for t in range(n_tok):
+        got = y[t * ys:t * ys + rows]
+        assert np.array_equal(got.view(np.uint32), want[t * ys:t * ys + rows].view(np.uint32)), t
+    wt.free()
