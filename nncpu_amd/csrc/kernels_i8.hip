@@ -23,56 +23,55 @@ namespace {
 
 // Eight lanes per block of 32 values, four values a lane: the block's maximum
 // and quant sum are three DPP steps each (a lane per value took ten LDS-crossbar
-// exchanges and four times the scale arithmetic per value: VALU-bound, 10.8 us
-// at 512 vectors of 3584 in the kernel trace, 6.3 this way).
-//   TK = 8, K = 4: a wave takes 8 vectors x 4 consecutive blocks (every load and
-//     store a whole 128- or 32-byte run), its loads in flight together; from
-//     QUANT_TILE_MIN vectors.
-//   TK = 1, K = 1: a wave takes 8 consecutive blocks; few vectors (latency).
+// exchanges and four times the scale arithmetic per value, which bound it).
+//   TILE8: a wave takes one block of 8 vectors, a workgroup 4 blocks of 8, so
+//     the block-major scales are written in runs; from QUANT_TILE_MIN vectors.
+//     (Four blocks a lane, whose loads would be in flight together, leave too few
+//     waves: 1.0 to 2.8 us more at 17 to 512 vectors of 1024 to 18944.)
+//   otherwise a wave takes 8 consecutive blocks; few vectors.
+// Quantizing and multiplying by a 256-row Q8_0 matrix, us, with a lane per value
+// and now: 17 vectors of 2048 21.2 / 21.0, 512 of 3584 34.6 / 30.3, 512 of 18944
+// 79.6 / 59.6.
 constexpr int QUANT_TILE_MIN = 17;
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
-template <int TK, int K>
+template <bool TILE8>
 __global__ __launch_bounds__(256) void quantize_act_kernel(const float* __restrict__ x, size_t x_stride, int cols,
                                                            int n_tok, int8_t* __restrict__ q,
                                                            uint16_t* __restrict__ s, double* __restrict__ sx,
                                                            float* __restrict__ sxT, int tok_pad) {
     const int nb = cols >> 5, p = threadIdx.x & 7, grp = threadIdx.x >> 3;
-    int t, b0;
-    if (TK == 8) {
-        t = blockIdx.y * 8 + (grp & 7);
-        b0 = (blockIdx.x * 4 + (grp >> 3)) * K;
+    int t, b;
+    if (TILE8) {
+        const int gx = (nb + 3) >> 2;  // workgroups along the blocks (one-dimensional grid: any number of vectors)
+        t = blockIdx.x / gx * 8 + (grp & 7);
+        b = blockIdx.x % gx * 4 + (grp >> 3);
     } else {
         const int blk = blockIdx.x * 32 + grp;
         t = blk / nb;
-        b0 = blk - t * nb;
+        b = blk - t * nb;
     }
-    const float* xr = x + (size_t)(t < n_tok ? t : n_tok - 1) * x_stride + 4 * p;  // loads stay in bounds; stores are skipped
-    f4u v[K];
+    // Loads stay in bounds; past the end the stores are skipped.
+    const f4u v = *(const f4u*)(x + (size_t)(t < n_tok ? t : n_tok - 1) * x_stride + 32 * (size_t)(b < nb ? b : nb - 1) +
+                                4 * p);
+    const float a = max8(fmaxf(fmaxf(q8_abs(v[0]), q8_abs(v[1])), fmaxf(q8_abs(v[2]), q8_abs(v[3]))));
+    const Q8Scale qs = q8_scale(a);
+    int qi[4];
 #pragma unroll
-    for (int k = 0; k < K; ++k) v[k] = *(const f4u*)(xr + 32 * (size_t)(b0 + k < nb ? b0 + k : nb - 1));
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-        const float a = max8(fmaxf(fmaxf(q8_abs(v[k][0]), q8_abs(v[k][1])), fmaxf(q8_abs(v[k][2]), q8_abs(v[k][3]))));
-        const Q8Scale qs = q8_scale(a);
-        int qi[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) qi[e] = q8_quant(v[k][e], qs.inv);
-        const int qsum = sum8(qi[0] + qi[1] + qi[2] + qi[3]);
-        const int b = b0 + k;
-        if (b >= nb || t >= n_tok) continue;
-        *(uint32_t*)(q + (size_t)t * cols + 32 * (size_t)b + 4 * p) =
-            (uint32_t)(qi[0] & 255) | (uint32_t)(qi[1] & 255) << 8 | (uint32_t)(qi[2] & 255) << 16 |
-            (uint32_t)(qi[3] & 255) << 24;
-        if (p == 0) {
-            const size_t i = (size_t)t * nb + b;
-            s[i] = (uint16_t)qs.bits;
-            *(double2*)(sx + 2 * i) = double2{(double)qs.scale, (double)qs.scale * (double)qsum};  // exact: s_x * sum(q_x)
-            // Block-major f32 copies for the GEMM: [b][tok_pad] scale, then [b][tok_pad] scale * sum(q).
-            if (sxT) {
-                sxT[(size_t)b * tok_pad + t] = qs.scale;
-                sxT[(size_t)nb * tok_pad + (size_t)b * tok_pad + t] = qs.scale * (float)qsum;  // exact: 8 + 13 bits
-            }
+    for (int e = 0; e < 4; ++e) qi[e] = q8_quant(v[e], qs.inv);
+    const int qsum = sum8(qi[0] + qi[1] + qi[2] + qi[3]);
+    if (b >= nb || t >= n_tok) return;
+    *(uint32_t*)(q + (size_t)t * cols + 32 * (size_t)b + 4 * p) =
+        (uint32_t)(qi[0] & 255) | (uint32_t)(qi[1] & 255) << 8 | (uint32_t)(qi[2] & 255) << 16 |
+        (uint32_t)(qi[3] & 255) << 24;
+    if (p == 0) {
+        const size_t i = (size_t)t * nb + b;
+        s[i] = (uint16_t)qs.bits;
+        *(double2*)(sx + 2 * i) = double2{(double)qs.scale, (double)qs.scale * (double)qsum};  // exact: s_x * sum(q_x)
+        // Block-major f32 copies for the GEMM: [b][tok_pad] scale, then [b][tok_pad] scale * sum(q).
+        if (sxT) {
+            sxT[(size_t)b * tok_pad + t] = qs.scale;
+            sxT[(size_t)nb * tok_pad + (size_t)b * tok_pad + t] = qs.scale * (float)qsum;  // exact: 8 + 13 bits
         }
     }
 }
@@ -980,10 +979,10 @@ void launch_quantize_act(const float* x, size_t x_stride, int cols, int n_tok, i
                          float* sxT, int tok_pad, hipStream_t st) {
     const int nb = cols / 32;
     if (n_tok >= QUANT_TILE_MIN)
-        quantize_act_kernel<8, 4><<<dim3(ceil_div(nb, 16), ceil_div(n_tok, 8)), 256, 0, st>>>(x, x_stride, cols, n_tok,
-                                                                                               q, s, sx, sxT, tok_pad);
+        quantize_act_kernel<true><<<ceil_div(nb, 4) * ceil_div(n_tok, 8), 256, 0, st>>>(x, x_stride, cols, n_tok, q, s, sx,
+                                                                                        sxT, tok_pad);
     else
-        quantize_act_kernel<1, 1><<<ceil_div((long)nb * n_tok, 32), 256, 0, st>>>(x, x_stride, cols, n_tok, q, s, sx,
+        quantize_act_kernel<false><<<ceil_div((long)nb * n_tok, 32), 256, 0, st>>>(x, x_stride, cols, n_tok, q, s, sx,
                                                                                    sxT, tok_pad);
 }
 

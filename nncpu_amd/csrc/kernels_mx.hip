@@ -89,15 +89,17 @@ __device__ __forceinline__ int mx_exponent(float amax) {
 }
 
 // Eight lanes per block of 32 values, four values a lane (max and sum: three DPP
-// steps each); a wave takes 8 tokens x 4 consecutive blocks, so its loads are
-// 128-byte runs in flight together and its BF16 stores whole runs of the tiled
-// layout (a half-wave per block, a value a lane: VALU-bound, 42 us at 512 tokens
-// of 18944 and 10.7 of 3584 in the kernel trace, 14.8 and 6.4 this way). Blocks past nb (up to the group-padded nbp8) and
-// tokens past n_tok (up to xl_tok, whole GEMM token tiles) only write zeros: the
-// limbs of xl, and for tokens past n_tok the xb values. PARTS: which parts of
-// the buffer are written (MxParts).
+// steps each; a lane per value took ten LDS-crossbar exchanges and was bound by
+// them); a workgroup takes 4 blocks of 8 tokens, its BF16 stores whole runs of
+// the tiled layout. Four blocks a lane measured the same at long rows of 18944
+// and 1 to 2 us slower at 1024 to 3584 (too few waves). Quantizing and
+// multiplying by a 256-row Q8_0 matrix, us, with a lane per value and now: 512
+// tokens of 3584 32.4 / 28.3, 512 of 18944 72.7 / 48.6, 17 of 2048 23.8 / 23.8.
+// Blocks past nb (up to the group-padded nbp8) and tokens past n_tok (up to
+// xl_tok, whole GEMM token tiles) only write zeros: the limbs of xl, and for
+// tokens past n_tok the xb values. PARTS: which parts of the buffer are written
+// (MxParts).
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-constexpr int MXQ_K = 4;  // blocks per thread
 
 template <int PARTS>
 __global__ __launch_bounds__(256) void quantize_mx_kernel(const float* __restrict__ x, size_t x_stride, int cols,
@@ -107,53 +109,48 @@ __global__ __launch_bounds__(256) void quantize_mx_kernel(const float* __restric
                                                           uint16_t* __restrict__ xb, uint16_t* __restrict__ xl) {
     constexpr bool INT8 = PARTS & MX_PART_INT8, GEMM = PARTS & MX_PART_GEMM;
     const int nb = cols >> 5, p = threadIdx.x & 7, grp = threadIdx.x >> 3;
-    const int t = blockIdx.y * 8 + (grp & 7), b0 = (blockIdx.x * 4 + (grp >> 3)) * MXQ_K;  // xl_tok, nbp8: multiples of 8
-    const float* xr = x + (size_t)(t < n_tok ? t : n_tok - 1) * x_stride + 4 * p;  // loads stay in bounds
-    f4u v[MXQ_K];
-#pragma unroll
-    for (int k = 0; k < MXQ_K; ++k) v[k] = *(const f4u*)(xr + 32 * (size_t)(b0 + k < nb ? b0 + k : nb - 1));
+    const int gx = nbp8 >> 2;  // workgroups along the blocks (one-dimensional grid: any number of vectors)
+    const int t = blockIdx.x / gx * 8 + (grp & 7), b = blockIdx.x % gx * 4 + (grp >> 3);  // xl_tok, nbp8: multiples of 8
+    const f4u v = *(const f4u*)(x + (size_t)(t < n_tok ? t : n_tok - 1) * x_stride + 32 * (size_t)(b < nb ? b : nb - 1) +
+                                4 * p);  // in bounds
     // xb tiled: [token tile][block][token in tile][32], 16-byte chunks of a
     // row swizzled as the GEMM's LDS rows are (chunk c at c ^ ((row >> 2) & 3)).
     const int tt = t / MX_TM_Q, tr = t % MX_TM_Q;
     uint16_t* xw = xb + ((size_t)tt * nb * MX_TM_Q + tr) * 32 + (((p >> 1) ^ ((tr >> 2) & 3)) << 3) + 4 * (p & 1);
+    // amax over the block, NaN skipped (as nncpu's encoder's `v.abs() > amax`).
+    const float a = max8(fmaxf(fmaxf(q8_abs(v[0]), q8_abs(v[1])), fmaxf(q8_abs(v[2]), q8_abs(v[3]))));
+    const bool zero = !(a > 0.0f);
+    const int E = mx_exponent(a);
+    const float scale = zero ? 0.0f : __uint_as_float((uint32_t)(E + 127) << 23);
+    int qi[4];
+    uint32_t w[4];
 #pragma unroll
-    for (int k = 0; k < MXQ_K; ++k) {
-        // amax over the block, NaN skipped (as nncpu's encoder's `v.abs() > amax`).
-        const float a = max8(fmaxf(fmaxf(q8_abs(v[k][0]), q8_abs(v[k][1])), fmaxf(q8_abs(v[k][2]), q8_abs(v[k][3]))));
-        const bool zero = !(a > 0.0f);
-        const int E = mx_exponent(a);
-        const float scale = zero ? 0.0f : __uint_as_float((uint32_t)(E + 127) << 23);
-        int qi[4];
-        uint32_t w[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int r = zero ? 0 : rint_sat(__builtin_ldexpf(v[k][e], -E));  // v 2^-E: exact unless below 2^-126 (then |q| < 1)
-            qi[e] = r < -127 ? -127 : (r > 127 ? 127 : r);
-            w[e] = __float_as_uint((float)qi[e] * scale) >> 16;  // q 2^E as BF16: at most 7 significant bits
-        }
-        const int qsum = sum8(qi[0] + qi[1] + qi[2] + qi[3]);
-        const int b = b0 + k;
-        if (b >= nbp8 || t >= xl_tok) continue;
-        const bool in = b < nb && t < n_tok;
-        if (GEMM && b < nb)
-            *(uint2*)(xw + (size_t)b * MX_TM_Q * 32) = in ? make_uint2(w[0] | w[1] << 16, w[2] | w[3] << 16) : uint2{0, 0};
-        if (INT8 && in)
-            *(uint32_t*)(q + (size_t)t * cols + 32 * (size_t)b + 4 * p) =
-                (uint32_t)(qi[0] & 255) | (uint32_t)(qi[1] & 255) << 8 | (uint32_t)(qi[2] & 255) << 16 |
-                (uint32_t)(qi[3] & 255) << 24;
-        if (p == 0) {
-            const float X = scale * (float)qsum;  // exact: <= 12 significant bits
-            // X = hi + lo, hi its top 8 significant bits, lo the rest (<= 4 bits).
-            const uint32_t hb = __float_as_uint(X) & 0xFFFF0000u;
-            const float lo = X - __uint_as_float(hb);
-            if (GEMM) *(uint32_t*)(xl + ((size_t)t * nbp8 + b) * 2) = in ? (hb >> 16) | (__float_as_uint(lo) & 0xFFFF0000u) : 0u;
-            if (INT8 && in) {
-                const size_t i = (size_t)t * nb + b;
-                s[i] = (uint16_t)(__float_as_uint(scale) >> 16);
-                *(double2*)(sx + 2 * i) = double2{(double)scale, (double)X};
-                sxT[(size_t)b * tok_pad + t] = scale;
-                sxT[(size_t)nb * tok_pad + (size_t)b * tok_pad + t] = X;
-            }
+    for (int e = 0; e < 4; ++e) {
+        const int r = zero ? 0 : rint_sat(__builtin_ldexpf(v[e], -E));  // v 2^-E: exact unless below 2^-126 (then |q| < 1)
+        qi[e] = r < -127 ? -127 : (r > 127 ? 127 : r);
+        w[e] = __float_as_uint((float)qi[e] * scale) >> 16;  // q 2^E as BF16: at most 7 significant bits
+    }
+    const int qsum = sum8(qi[0] + qi[1] + qi[2] + qi[3]);
+    if (t >= xl_tok) return;
+    const bool in = b < nb && t < n_tok;
+    if (GEMM && b < nb)
+        *(uint2*)(xw + (size_t)b * MX_TM_Q * 32) = in ? make_uint2(w[0] | w[1] << 16, w[2] | w[3] << 16) : uint2{0, 0};
+    if (INT8 && in)
+        *(uint32_t*)(q + (size_t)t * cols + 32 * (size_t)b + 4 * p) =
+            (uint32_t)(qi[0] & 255) | (uint32_t)(qi[1] & 255) << 8 | (uint32_t)(qi[2] & 255) << 16 |
+            (uint32_t)(qi[3] & 255) << 24;
+    if (p == 0) {
+        const float X = scale * (float)qsum;  // exact: <= 12 significant bits
+        // X = hi + lo, hi its top 8 significant bits, lo the rest (<= 4 bits).
+        const uint32_t hb = __float_as_uint(X) & 0xFFFF0000u;
+        const float lo = X - __uint_as_float(hb);
+        if (GEMM) *(uint32_t*)(xl + ((size_t)t * nbp8 + b) * 2) = in ? (hb >> 16) | (__float_as_uint(lo) & 0xFFFF0000u) : 0u;
+        if (INT8 && in) {
+            const size_t i = (size_t)t * nb + b;
+            s[i] = (uint16_t)(__float_as_uint(scale) >> 16);
+            *(double2*)(sx + 2 * i) = double2{(double)scale, (double)X};
+            sxT[(size_t)b * tok_pad + t] = scale;
+            sxT[(size_t)nb * tok_pad + (size_t)b * tok_pad + t] = X;
         }
     }
 }
@@ -738,9 +735,10 @@ void launch_quantize_mx(const float* x, size_t x_stride, int cols, int n_tok, in
                         float* sxT, int tok_pad, uint16_t* xb, uint16_t* xl, int parts, hipStream_t st) {
     const int nbp8 = mx_nbp8(cols / 32), xl_tok = mx_xl_tok(n_tok);
     // Without the GEMM's parts no token past n_tok is touched.
-    const dim3 grid(ceil_div(nbp8, 4 * MXQ_K), parts == MX_PART_INT8 ? ceil_div(n_tok, 8) : xl_tok / 8);
-#define NNH_Q(P) \
-    quantize_mx_kernel<P><<<grid, 256, 0, st>>>(x, x_stride, cols, n_tok, nbp8, q, s, sx, sxT, tok_pad, xl_tok, xb, xl)
+    const int groups = parts == MX_PART_INT8 ? ceil_div(n_tok, 8) : xl_tok / 8;
+#define NNH_Q(P)                                                                                                     \
+    quantize_mx_kernel<P><<<nbp8 / 4 * groups, 256, 0, st>>>(x, x_stride, cols, n_tok, nbp8, q, s, sx, sxT, tok_pad, \
+                                                             xl_tok, xb, xl)
     if (parts == MX_PART_INT8)
         NNH_Q(MX_PART_INT8);
     else if (parts == MX_PART_GEMM)

@@ -58,3 +58,21 @@ def test_batched_quantizer_bits(oracle, act, cols, n_tok, pad):
     sxt = b[off_t:off_t + 8 * nb * pad_tok].view(np.float32).reshape(2, nb, pad_tok)[:, :, :n_tok]
     assert np.array_equal(sxt[0].T[fin], scale[fin].astype(np.float32))
     assert np.array_equal(sxt[1].T[fin], (scale * total)[fin].astype(np.float32))
+
+
+@pytest.mark.parametrize("act", [1, 2])
+def test_more_vectors_than_a_grid_dimension_holds(act):
+    """8 * 65535 vectors and more: the last ones are quantized as they are alone."""
+    import torch
+    cols, n_tok = 32, 8 * 65536 + 9
+    x = torch.randn(n_tok, cols, device="cuda")
+    bufs = []
+    for first in (0, n_tok - 20):
+        off_s, off_sx, size = N.act_layout_ex(act, cols, n_tok - first)
+        buf = torch.zeros(size, dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        N.quantize_act_ex_dev(act, x[first:].data_ptr(), cols, cols, n_tok - first, buf.data_ptr())
+        N.sync()
+        q, s = buf[:(n_tok - first) * cols], buf[off_s:off_s + 2 * (n_tok - first)]
+        bufs.append((q[-20 * cols:].cpu(), s[-40:].cpu()))
+    assert torch.equal(bufs[0][0], bufs[1][0]) and torch.equal(bufs[0][1], bufs[1][1])
