@@ -1,0 +1,121 @@
+"""The int8 GEMM where its tiles are not whole rounds of the CUs: the last round
+is split along K (one spare tile, half a round, rounds that the split does not
+take), against the exact sum of the quantized product; a capped scratch keeps the
+tail whole; and scratch reserved for a batch serves smaller ones under capture."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+N = pytest.importorskip("nncpu_amd")
+
+
+@pytest.fixture(scope="module", autouse=True)
+def device():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    N.init(0)
+
+
+def matrix(dtype, rows, cols, seed):
+    rng = np.random.default_rng(seed)
+    nb = cols // 32
+
+    def bf16(a):
+        return (a.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+
+    s = bf16(rng.uniform(1e-4, 4e-4, (rows, nb)))
+    if dtype == 1:
+        q = rng.integers(-127, 128, (rows, cols), dtype=np.int8)
+        return (q, s), N.Weight.q8_0(q, s.view(np.int16), rows, cols)
+    q, b = rng.integers(0, 256, (rows, cols // 2), dtype=np.uint8), bf16(rng.uniform(-4e-3, 4e-3, (rows, nb)))
+    return (q, s, b), N.Weight.q4(q, s.view(np.int16), b.view(np.int16), rows, cols)
+
+
+def run(w, x, call=None):
+    import torch
+    n, cols = x.shape
+    y = torch.empty(n, w.rows(), device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    w.prepare(N.ACT_I8, n)
+    (call or N.gemv_batch_dev)(w, x.data_ptr(), cols, y.data_ptr(), w.rows(), n, N.ACT_I8, st)
+    torch.cuda.synchronize()
+    return y
+
+
+@pytest.mark.parametrize("dtype", [1, 2])
+@pytest.mark.parametrize("rows,cols,n_tok", [
+    (85 * 128 + 1, 2048, 300),   # 258 tiles: 2 left, 8 splits
+    (97 * 128 - 5, 1504, 500),   # 388 tiles: 132 left, one split: the round stays whole
+    (96 * 128, 3104, 512),       # 384 tiles: 128 left, 2 splits of 97 blocks
+    (256 * 128, 1600, 100),      # a whole round
+])
+def test_split_tail(dtype, rows, cols, n_tok):
+    import torch
+    parts, w = matrix(dtype, rows, cols, rows + cols)
+    nb = cols // 32
+    g = torch.Generator(device="cuda")
+    g.manual_seed(rows)
+    x = torch.randn(n_tok, cols, generator=g, device="cuda")
+    y = run(w, x)
+    w.free()
+    off_s, _, size = N.act_layout_ex(N.ACT_I8, cols, n_tok)
+    buf = torch.zeros(size, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    N.quantize_act_ex_dev(N.ACT_I8, x.data_ptr(), cols, cols, n_tok, buf.data_ptr())
+    N.sync()
+    qx = buf[:n_tok * cols].view(torch.int8).view(n_tok, nb, 32).double()
+    sx = buf[off_s:off_s + 2 * n_tok * nb].view(torch.bfloat16).view(n_tok, nb, 1).double()
+    q, s = torch.from_numpy(parts[0]).cuda(), torch.from_numpy(parts[1].view(np.int16)).cuda().view(torch.bfloat16)
+    if dtype == 2:
+        q = q.view(rows, nb, 16)
+        q = torch.cat([q & 15, q >> 4], 2)
+    wd = q.view(rows, nb, 32).double() * s.double().unsqueeze(2)
+    if dtype == 2:
+        wd = wd + torch.from_numpy(parts[2].view(np.int16)).cuda().view(torch.bfloat16).double().unsqueeze(2)
+    exact = (qx * sx).view(n_tok, cols) @ wd.view(rows, cols).T.contiguous()
+    # Groups of 8 blocks are summed in f32 (Q4: two terms a block), everything else
+    # in f64 and rounded once: 8 (16) roundings of at most the groups' magnitude.
+    mag = (qx * sx).abs().view(n_tok, cols) @ wd.abs().view(rows, cols).T.contiguous()
+    if dtype == 2:  # quant and bias terms one by one: |q s| + |bias| <= 0..15 s + |bias|
+        up = q.view(rows, nb, 32).double() * s.double().unsqueeze(2) + torch.from_numpy(
+            parts[2].view(np.int16)).cuda().view(torch.bfloat16).double().abs().unsqueeze(2)
+        mag = (qx * sx).abs().view(n_tok, cols) @ up.view(rows, cols).T.contiguous()
+    bound = (8 if dtype == 1 else 16) * 2.0 ** -24 * mag + 2.0 ** -24 * exact.abs()
+    assert bool(((y.double() - exact).abs() <= bound).all())
+
+
+def test_capped_scratch_keeps_the_tail_whole():
+    """The fixed scratch (64 MiB) has no room for these activations and a split tail: the call is taken all the same."""
+    import torch
+    rows, cols, n_tok = 30 * 128, 18944, 1100  # 270 tiles
+    _, w = matrix(2, rows, cols, 5)
+    x = torch.randn(n_tok, cols, device="cuda")
+    a, b = run(w, x), run(w, x, N.gemv_batch_dev_noalloc)
+    assert float((a.double() - b.double()).norm() / a.double().norm()) < 2e-7  # each within about 6e-8 of the exact sum
+    w.free()
+
+
+def test_reserved_stream_serves_smaller_batches_under_capture():
+    import torch
+    rows, cols = 86 * 128, 2048
+    _, w = matrix(1, rows, cols, 6)
+    x = torch.randn(768, cols, device="cuda")
+    eager = run(w, x[:384])  # 258 tiles, a split tail
+    st = torch.cuda.Stream()
+    N.stream_reserve(w, N.ACT_I8, 768, st.cuda_stream)
+    y = torch.empty(384, rows, device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        N.gemv_batch_dev(w, x.data_ptr(), cols, y.data_ptr(), rows, 384, N.ACT_I8, st.cuda_stream)
+    for _ in range(3):
+        y.fill_(0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, eager)
+    del graph
+    N.stream_release(st.cuda_stream)
+    w.free()
