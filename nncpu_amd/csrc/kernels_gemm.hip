@@ -14,10 +14,9 @@
 // total every 8 blocks (an f32 sum over K = 18944 would take most of the
 // 1e-5 tolerance next to nncpu's own f32 rounding; chunks of 8 keep the
 // error within 8 f32 roundings of the absolute block terms). The scale
-// products s_w[n] s_x[m] come from the matrix unit too: one
-// v_mfma_f32_32x32x1_2b_f32 forms the outer products of two blocks exactly,
-// already in the result layout, so each lane needs one scale per block
-// instead of sixteen; and the Q4 bias term sum_b bias[n,b] (s_x sum q_x)[m,b]
+// products s_w[n] s_x[m] come from the matrix unit too: a BF16 MFMA forms the
+// outer products exactly, already in the result layout, so each lane needs one
+// scale per block instead of sixteen; and the Q4 bias term sum_b bias[n,b] (s_x sum q_x)[m,b]
 // is an outer-product sum, one v_mfma_f32_32x32x2f32 per two blocks
 // accumulating into the same f32 tile. nncpu's per-32 BF16 scales make this
 // epilogue, not the int8 MFMA, the compute bound: 2 VALU ops per output and
@@ -151,14 +150,33 @@ __device__ __forceinline__ void issue_stage(GStage<DT, KB>& st, const GArgs& g, 
     }
 }
 
-// Two outer products u_0 v_0^T and u_1 v_1^T of 32-vectors, exact in f32
-// (the factors are BF16 values, so every product has at most 16 significant
-// bits), each laid out like the i8 MFMA's result: one
-// v_mfma_f32_32x32x1_2b_f32, lane l giving u_{l/32}[l%32] and v_{l/32}[l%32];
-// result registers 16 b .. 16 b + 15 hold product b.
+// Outer products u v^T of 32-vectors of BF16 values (given as f32), on the BF16
+// matrix unit, each laid out like the i8 MFMA's result. A product of two BF16
+// values has at most 16 significant bits, so it is exact in f32 (subnormal
+// factors and products included: checked against the f32 unit's bits over
+// scales from the smallest subnormal to infinity and NaN); the other K slots
+// hold 0 * 0. BF16 because vector instructions run beside it, which they do not
+// beside f32 matrix instructions (measured for both forms, against
+// v_mfma_f32_32x32x1_2b: Q8_0 18944 x 3584, 512 vectors 149 -> 140 us, Q4
+// 170 -> 165).
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ int bf16_bits(float v) { return (int)(__float_as_uint(v) >> 16); }
+
+// Both products of a pair of blocks: lane l gives u_{l/32}[l%32] and
+// v_{l/32}[l%32], result registers 16 b .. 16 b + 15 hold product b.
 __device__ __forceinline__ v32f outer32x2(float u, float v) {
     const v32f z = {};
-    return __builtin_amdgcn_mfma_f32_32x32x1f32(u, v, z, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x4bf16_1k(v4s{(short)bf16_bits(u), 0, 0, 0}, v4s{(short)bf16_bits(v), 0, 0, 0},
+                                                    z, 0, 0, 0);
+}
+
+// One product, of the lanes that are `on` (one half of the wave).
+__device__ __forceinline__ v16f outer32(int u, int v, bool on) {
+    const v16f z = {};
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8b, v4i{on ? u : 0, 0, 0, 0}),
+                                                   __builtin_bit_cast(v8b, v4i{on ? v : 0, 0, 0, 0}), z, 0, 0, 0);
 }
 
 // One wave's 32 x 32 tile (rows rowA.., tokens colB..) over the stage's
@@ -173,7 +191,12 @@ __device__ __forceinline__ void compute_stage(const GStage<DT, KB>& st, v16f& ac
     for (int jp = 0; jp < KB; jp += 2) {
         if (jp >= nblk) break;
         const int jh = jp + h;  // this lane's block for the scale products
-        const v32f S = outer32x2(st.SW[jh * TILE + rowA + c], st.SX[jh * TILE + colB + c]);  // s_w[n] s_x[m]
+        const float sw = st.SW[jh * TILE + rowA + c], sx = st.SX[jh * TILE + colB + c];
+        // s_w[n] s_x[m]: Q8 both blocks' at once; Q4, whose bias operands need
+        // registers too, a block's at a time (both: 2 VGPRs spilled, 176 us
+        // against 165 at the size above; Q8 one at a time 148 against 140).
+        v32f S2;
+        if (DT == 1) S2 = outer32x2(sw, sx);
 #pragma unroll
         for (int jj = 0; jj < 2; ++jj) {
             const int j = jp + jj;
@@ -190,11 +213,13 @@ __device__ __forceinline__ void compute_stage(const GStage<DT, KB>& st, v16f& ac
                 a.z = (int)((unsigned)q.z >> sh) & mk;
                 a.w = (int)((unsigned)q.w >> sh) & mk;
             }
+            v16f S;
+            if (DT == 2) S = outer32(bf16_bits(sw), bf16_bits(sx), h == jj);
             const v16i z = {};
             const v16i P = __builtin_amdgcn_mfma_i32_32x32x32_i8(v4i{a.x, a.y, a.z, a.w}, v4i{bq.x, bq.y, bq.z, bq.w},
                                                                  z, 0, 0, 0);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[r] = __builtin_fmaf((float)P[r], S[16 * jj + r], acc[r]);
+            for (int r = 0; r < 16; ++r) acc[r] = __builtin_fmaf((float)P[r], DT == 1 ? S2[16 * jj + r] : S[r], acc[r]);
         }
         if (DT == 2) {
             // Bias term of the pair: acc += sum_j bias[n, j] (s_x sum q_x)[m, j],
