@@ -157,8 +157,9 @@ __device__ __forceinline__ void issue_stage(GStage<DT, KB>& st, const GArgs& g, 
 // scales from the smallest subnormal to infinity and NaN); the other K slots
 // hold 0 * 0. BF16 because vector instructions run beside it, which they do not
 // beside f32 matrix instructions (measured for both forms, against
-// v_mfma_f32_32x32x1_2b: Q8_0 18944 x 3584, 512 vectors 149 -> 140 us, Q4
-// 170 -> 165).
+// v_mfma_f32_32x32x1_2b, two runs each: Q8_0 18944 x 3584, 512 vectors 150 / 151
+// -> 145 / 144 us, 3584 x 18944 157 / 159 -> 148 / 150; Q4 18944 x 3584 172 / 175
+// -> 172 / 172).
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef __bf16 v8b __attribute__((ext_vector_type(8)));
 
@@ -193,8 +194,8 @@ __device__ __forceinline__ void compute_stage(const GStage<DT, KB>& st, v16f& ac
         const int jh = jp + h;  // this lane's block for the scale products
         const float sw = st.SW[jh * TILE + rowA + c], sx = st.SX[jh * TILE + colB + c];
         // s_w[n] s_x[m]: Q8 both blocks' at once; Q4, whose bias operands need
-        // registers too, a block's at a time (both: 2 VGPRs spilled, 176 us
-        // against 165 at the size above; Q8 one at a time 148 against 140).
+        // registers too, a block's at a time (both: 2 VGPRs spilled, 7 % slower
+        // at the size above; Q8 one at a time 6 % slower).
         v32f S2;
         if (DT == 1) S2 = outer32x2(sw, sx);
 #pragma unroll
