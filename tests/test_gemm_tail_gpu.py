@@ -86,6 +86,26 @@ def test_split_tail(dtype, rows, cols, n_tok):
     assert bool(((y.double() - exact).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("dtype", [1, 2])
+@pytest.mark.parametrize("rows,cols,n_tok,roll", [
+    (86 * 128, 2048, 384, 128),         # 258 tiles: 2 left, 8 splits
+    (84 * 128, 3584, 512, 20 * 128),    # 336 tiles: 80 left, 3 splits of 14 groups of 8 blocks
+    (96 * 128 - 9, 3200, 500, 32 * 128),  # 384 tiles: 128 left, 2 splits of 12 groups and a half
+])
+def test_split_tail_keeps_the_bits(dtype, rows, cols, n_tok, roll):
+    """The tail's rows are computed whole when they are the matrix's first ones: the same bits."""
+    import torch
+    parts, w = matrix(dtype, rows, cols, rows + n_tok)
+    make = N.Weight.q8_0 if dtype == 1 else N.Weight.q4
+    turned = [np.roll(p.reshape(rows, -1), roll, axis=0) for p in parts]
+    wt = make(*[p if i == 0 else p.view(np.int16) for i, p in enumerate(turned)], rows, cols)
+    x = torch.randn(n_tok, cols, device="cuda")
+    y, yt = run(w, x), run(wt, x)
+    assert torch.equal(y, yt.roll(-roll, 1))
+    w.free()
+    wt.free()
+
+
 def test_capped_scratch_keeps_the_tail_whole():
     """The fixed scratch (64 MiB) has no room for these activations and a split tail: the call is taken all the same."""
     import torch
