@@ -86,6 +86,13 @@ __device__ __forceinline__ void wait_vm_keep(const void* a = nullptr, const void
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(K), "s"(a), "s"(b), "s"(c) : "memory");
 }
 
+// The instruction of every direct-to-LDS copy that is written as asm. The copy
+// reads its LDS address from M0, and one wait state is required between a
+// scalar write of M0 and such a load. The compiler writes M0 right before the
+// asm and inserts the wait state for the builtin only, since it cannot see the
+// load in here; without it a copy may land at the previous copy's address.
+#define NNH_COPY16_ASM "s_nop 0\n\tglobal_load_lds_dwordx4 "
+
 // One 1 KB copy of the bytes [off, off + 1024) of a span of `len` bytes
 // (a multiple of 16) to dst (uniform); lanes past the end repeat the span's
 // last 16 bytes. Issued as asm: for the builtin the compiler cannot tell
@@ -94,7 +101,7 @@ __device__ __forceinline__ void wait_vm_keep(const void* a = nullptr, const void
 // explicit instead).
 __device__ __forceinline__ void copy_1k(const void* span, size_t len, size_t off, unsigned char* dst, int lane) {
     const size_t o = min(off + lane * 16, len - 16);
-    asm volatile("global_load_lds_dwordx4 %0, off" ::"v"((const unsigned char*)span + o),
+    asm volatile(NNH_COPY16_ASM "%0, off" ::"v"((const unsigned char*)span + o),
                  "{m0}"((uint32_t)(uintptr_t)dst)
                  : "memory");
 }

@@ -58,7 +58,7 @@ struct BatchArgs {
 // lane l's bytes at dst + 16 l); asm because the compiler would otherwise
 // drain every copy before any LDS read (the waits are explicit).
 __device__ __forceinline__ void copy16(const void* base, uint32_t voff, uint32_t dst) {
-    asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "{m0}"(dst) : "memory");
+    asm volatile(NNH_COPY16_ASM "%0, %1" ::"v"(voff), "s"(base), "{m0}"(dst) : "memory");
 }
 
 template <int N>

@@ -270,7 +270,7 @@ __device__ __forceinline__ MxLane mx_lane(const MxArgs& g, int wave, int lane) {
 // flight before each stage's first LDS read; the waits are explicit instead
 // (wait_vm, then a barrier).
 __device__ __forceinline__ void lds_load(const void* base, uint32_t voff, void* dst) {
-    asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "{m0}"((uint32_t)(uintptr_t)dst)
+    asm volatile(NNH_COPY16_ASM "%0, %1" ::"v"(voff), "s"(base), "{m0}"((uint32_t)(uintptr_t)dst)
                  : "memory");
 }
 

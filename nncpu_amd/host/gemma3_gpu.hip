@@ -362,7 +362,7 @@ __host__ int phase_chunks(const PkArgs& a, const F32Mat* w7, int phase, int mw) 
 // dst uniform). As asm, so the compiler neither waits for it nor reorders
 // LDS reads around it; the waits are explicit.
 __device__ __forceinline__ void copy16(const uint8_t* src, uint32_t dst) {
-    asm volatile("global_load_lds_dwordx4 %0, off" ::"v"(src), "{m0}"(dst) : "memory");
+    asm volatile(NNH_COPY16_ASM "%0, off" ::"v"(src), "{m0}"(dst) : "memory");
 }
 
 // Loader wave lw issues exactly k copy instructions for a phase's runs
