@@ -261,11 +261,12 @@ size_t nnh_argmax_work_bytes(size_t n);
 int nnh_argmax_dev(const float* v, size_t n, void* work, uint64_t* out_row, void* stream);
 
 /* nnh_gemv_batch_dev for callers that cannot allocate (code under HIP graph
- * capture, tight serving loops, harnesses that forbid hipMalloc): no
- * counterpart in the reference. Its scratch (Q4 block sums, quantized
+ * capture, tight serving loops, harnesses that forbid hipMalloc), with the
+ * same bits: no counterpart in the reference. Its scratch (Q4 block sums, quantized
  * activations, split-K partials) is one device array of
  * NNH_NOALLOC_SCRATCH_BYTES that the library holds on each GPU for the life
- * of the process; the call allocates nothing. Preconditions beyond
+ * of the process (32 MiB more hold the partial sums of the int8 GEMM's last
+ * tiles, which do not count below); the call allocates nothing. Preconditions beyond
  * nnh_gemv_batch_dev's: nnh_init has run, and the weight's layouts for this
  * (act, n_tok) exist (nnh_weight_prepare, or an earlier nnh_gemv_batch_dev
  * call), else NNH_E_STATE; a call needing more scratch than the maximum

@@ -66,8 +66,9 @@ size_t g_pinned_bytes = 0;
 // allocate: a device array each GPU holds for the process's lifetime, at its
 // own address, looked up once per device at init (g_noalloc). Host code
 // never passes the array's name to a kernel or copy: in host code it is a
-// stand-in, not a device address.
-static __device__ __align__(256) uint8_t scratch[NNH_NOALLOC_SCRATCH_BYTES];
+// stand-in, not a device address. The int8 GEMM's split tail has room of its
+// own, so that it is split here whenever nnh_gemv_batch_dev splits it.
+static __device__ __align__(256) uint8_t scratch[NNH_NOALLOC_SCRATCH_BYTES + nnh::GEMM_TAIL_BYTES];
 uint8_t* g_noalloc = nullptr;  // device address of `scratch` on g_device
 
 int fail(int code, const std::string& msg) {
@@ -198,11 +199,11 @@ constexpr size_t SKINNY_MIN_TOKENS = 4;
 constexpr size_t GEMM_MIN_TOKENS = 17;
 
 // Device workspace the int8 matmul needs beyond the activation buffer.
-size_t i8_workspace_bytes(const nnh_weight* w, size_t n_tok, int act, bool split_tail = true) {
+size_t i8_workspace_bytes(const nnh_weight* w, size_t n_tok, int act) {
     if (n_tok >= GEMM_MIN_TOKENS && act == NNH_ACT_MXI8)
         return nnh::gemm_mx_workspace_bytes((int)w->rows, (int)w->nb, (int)n_tok);
     if (n_tok >= GEMM_MIN_TOKENS)
-        return nnh::gemm_workspace_bytes((int)w->rows, (int)w->nb, (int)n_tok, split_tail);
+        return nnh::gemm_workspace_bytes((int)w->rows, (int)w->nb, (int)n_tok);
     if (n_tok >= SKINNY_MIN_TOKENS) return nnh::skinny_workspace_bytes((int)w->rows, (int)w->nb);
     return 0;
 }
@@ -211,7 +212,7 @@ size_t i8_workspace_bytes(const nnh_weight* w, size_t n_tok, int act, bool split
 // buffers start with the same q / s / sx / sxT, so every kernel but the MX
 // GEMM reads either.
 void launch_i8(const nnh_weight* w, int mode, const uint8_t* act, size_t n_tok, float* y, size_t y_stride,
-               uint8_t* ws, bool split_tail, hipStream_t st) {
+               uint8_t* ws, hipStream_t st) {
     const ActLayout l = act_layout(w->cols, n_tok, mode);
     const int8_t* q = (const int8_t*)act;
     const double* sx = (const double*)(act + l.off_sx);
@@ -222,7 +223,7 @@ void launch_i8(const nnh_weight* w, int mode, const uint8_t* act, size_t n_tok, 
                             (float*)ws, st);
     else if (n_tok >= GEMM_MIN_TOKENS)
         nnh::launch_gemm_i8(w->dtype, w->qs, w->swT, q, sxT, (int)w->rows, (int)w->nb, (int)n_tok, y, y_stride,
-                            (double*)ws, split_tail, st);
+                            (double*)ws, st);
     else if (n_tok >= SKINNY_MIN_TOKENS)
         nnh::launch_skinny_i8(w->dtype, w->qs, w->swT, q, sxT, (int)w->rows, (int)w->nb, (int)n_tok, y, y_stride,
                               (double*)ws, st);
@@ -233,7 +234,7 @@ void launch_i8(const nnh_weight* w, int mode, const uint8_t* act, size_t n_tok, 
 
 // Queue the matmul for device x / y; `scratch` holds xsum or the act buffer.
 int run_gemv(const nnh_weight* w, const float* x, size_t x_stride, float* y, size_t y_stride, size_t n_tok, int act,
-             uint8_t* scratch, hipStream_t st, bool split_tail = true) {
+             uint8_t* scratch, hipStream_t st) {
     const int rows = (int)w->rows, nb = (int)w->nb;
     if (w->dtype == NNH_BF16) {
         if (!nnh::launch_gemm_bf16(w->bpath, (const uint16_t*)w->raw, rows, (int)w->cols, x, x_stride, (int)n_tok, y,
@@ -253,7 +254,7 @@ int run_gemv(const nnh_weight* w, const float* x, size_t x_stride, float* y, siz
         // Only this call's matmul reads the buffer, so what it does not read stays unwritten.
         launch_quantize(act, x, x_stride, w->cols, n_tok, scratch,
                         n_tok >= GEMM_MIN_TOKENS ? nnh::MX_PART_GEMM : nnh::MX_PART_INT8, st);
-        launch_i8(w, act, scratch, n_tok, y, y_stride, scratch + l.bytes, split_tail, st);
+        launch_i8(w, act, scratch, n_tok, y, y_stride, scratch + l.bytes, st);
     }
     NNH_HIP(hipGetLastError());
     return NNH_OK;
@@ -292,10 +293,16 @@ size_t argmax_work_bytes(const nnh_weight* w, int act) {
     return align_up(argmax_parts(w, act) * 8) + (argmax_fused(w, act) && w->dtype == NNH_Q4S ? w->nb * 4 : 0);
 }
 
-size_t gemv_scratch_bytes(const nnh_weight* w, size_t n_tok, int act, bool split_tail = true) {
+size_t gemv_scratch_bytes(const nnh_weight* w, size_t n_tok, int act) {
     if (w->dtype == NNH_BF16) return 0;
     if (act == NNH_ACT_F32) return w->dtype == NNH_Q4S ? align_up(n_tok * w->nb * 4) : 0;
-    return act_layout(w->cols, n_tok, act).bytes + i8_workspace_bytes(w, n_tok, act, split_tail);
+    return act_layout(w->cols, n_tok, act).bytes + i8_workspace_bytes(w, n_tok, act);
+}
+
+// The part of it that the int8 GEMM's split tail takes.
+size_t gemv_tail_bytes(const nnh_weight* w, size_t n_tok, int act) {
+    if (w->dtype == NNH_BF16 || act != NNH_ACT_I8 || n_tok < GEMM_MIN_TOKENS) return 0;
+    return nnh::gemm_tail_bytes((int)w->rows, (int)w->nb, (int)n_tok);
 }
 
 int check_call(const nnh_weight* w, size_t x_stride, size_t y_stride, size_t n_tok, int act) {
@@ -842,16 +849,14 @@ int nnh_gemv_batch_dev_noalloc(const nnh_weight* w, const float* x, size_t x_str
     if ((w->ready & need) != need)
         return fail(NNH_E_STATE, "gemv noalloc: the weight's layouts for this mode and batch are not built "
                                  "(nnh_weight_prepare, or one call of nnh_gemv_batch_dev, builds them)");
-    // The GEMM's tail stays whole where its partial tiles would not fit.
-    const bool split_tail = gemv_scratch_bytes(w, n_tok, act) <= (size_t)NNH_NOALLOC_SCRATCH_BYTES;
-    const size_t bytes = gemv_scratch_bytes(w, n_tok, act, split_tail);
+    const size_t bytes = gemv_scratch_bytes(w, n_tok, act) - gemv_tail_bytes(w, n_tok, act);
     if (bytes > (size_t)NNH_NOALLOC_SCRATCH_BYTES)
         return fail(NNH_E_INVALID, "gemv noalloc: this call needs " + std::to_string(bytes) +
                                        " bytes of scratch, more than the no-alloc maximum of " +
                                        std::to_string((size_t)NNH_NOALLOC_SCRATCH_BYTES));
     const size_t xs = n_tok > 1 ? x_stride : w->cols;
     const size_t ys = n_tok > 1 ? y_stride : w->rows;
-    return run_gemv(w, x, xs, y, ys, n_tok, act, g_noalloc, (hipStream_t)stream, split_tail);
+    return run_gemv(w, x, xs, y, ys, n_tok, act, g_noalloc, (hipStream_t)stream);
 }
 
 int nnh_act_layout_ex(int act, size_t cols, size_t n_tok, size_t* off_s, size_t* off_sx, size_t* bytes) {
@@ -901,7 +906,7 @@ int nnh_gemv_act_dev(const nnh_weight* w, int act, const void* buf, size_t n_tok
     if ((rc = prepare_locked(w, layouts_for(w, act, n_tok)))) return rc;
     const size_t wsb = i8_workspace_bytes(w, n_tok, act);
     if (wsb && (rc = scratch_locked((hipStream_t)stream, wsb, &ws))) return rc;
-    launch_i8(w, act, (const uint8_t*)buf, n_tok, y, n_tok > 1 ? y_stride : w->rows, ws, true, (hipStream_t)stream);
+    launch_i8(w, act, (const uint8_t*)buf, n_tok, y, n_tok > 1 ? y_stride : w->rows, ws, (hipStream_t)stream);
     NNH_HIP(hipGetLastError());
     return NNH_OK;
 }

@@ -209,15 +209,16 @@ void launch_dequantize(uint32_t type, const uint8_t* src, size_t n, float* dst, 
 int gemm_rows_pad(int rows);
 int gemm_tok_pad(int n_tok);
 void launch_gemm_scales(const uint16_t* sc, const uint16_t* bi, float* swT, int rows, int nb, hipStream_t st);
-// split_tail: the last, partial round of tiles over the CUs may be split along
-// K (the caller has the workspace that takes).
-size_t gemm_workspace_bytes(int rows, int nb, int n_tok, bool split_tail);  // split-K partials; 0 if unsplit
+size_t gemm_workspace_bytes(int rows, int nb, int n_tok);  // split-K partials; 0 if unsplit
+// Those of a last, partial round of tiles over the CUs; 0 if it is not split.
+constexpr size_t GEMM_TAIL_BYTES = (size_t)32 << 20;  // the most
+size_t gemm_tail_bytes(int rows, int nb, int n_tok);
 // int8 MFMA matmul for 5..16 vectors (kernels_skinny.hip).
 size_t skinny_workspace_bytes(int rows, int nb);  // K-split partials; 0 if unsplit
 void launch_skinny_i8(int dtype, const uint8_t* qs, const float* swT, const int8_t* aq, const float* sxT, int rows,
                       int nb, int n_tok, float* y, size_t y_stride, double* ws, hipStream_t st);
 void launch_gemm_i8(int dtype, const uint8_t* qs, const float* swT, const int8_t* aq, const float* sxT, int rows,
-                    int nb, int n_tok, float* y, size_t y_stride, double* ws, bool split_tail, hipStream_t st);
+                    int nb, int n_tok, float* y, size_t y_stride, double* ws, hipStream_t st);
 void launch_block_dots(int dtype, const uint8_t* qs, const int8_t* aq, int rows, int nb, int n_tok, int32_t* P,
                        hipStream_t st);
 // MX int8 path (kernels_mx.hip): power-of-two activation scales and the BF16

@@ -432,7 +432,7 @@ struct GemmShare {
     int full, tail, splits;
 };
 
-GemmShare gemm_share(int rows, int nb, int n_tok, bool split_tail) {
+GemmShare gemm_share(int rows, int nb, int n_tok) {
     const int tiles = ceil_div(rows, TILE) * ceil_div(n_tok, TILE);
     int most = nb / (2 * GEMM_KB);
     if (most > GEMM_MAX_SPLITS) most = GEMM_MAX_SPLITS;
@@ -444,23 +444,29 @@ GemmShare gemm_share(int rows, int nb, int n_tok, bool split_tail) {
     int sp = tail ? GEMM_CUS / tail : 1;
     if (sp > most) sp = most;
     const int longest = 8 * ceil_div(ceil_div(nb, 8), sp);  // blocks of the longest part (whole groups of 8)
-    if (split_tail && tiles > GEMM_CUS && sp > 1 && nb - longest >= GEMM_TAIL_BLOCKS) return {tiles - tail, tail, sp};
+    if (tiles > GEMM_CUS && sp > 1 && nb - longest >= GEMM_TAIL_BLOCKS) return {tiles - tail, tail, sp};
     return {0, tiles, 1};
 }
 
-size_t gemm_workspace_bytes(int rows, int nb, int n_tok, bool split_tail) {
-    constexpr size_t PART = (size_t)TILE * TILE * sizeof(double);
+constexpr size_t GEMM_PART = (size_t)TILE * TILE * sizeof(double);
+static_assert(GEMM_CUS * GEMM_PART == GEMM_TAIL_BYTES, "a split tail is at most one round of parts");
+
+size_t gemm_tail_bytes(int rows, int nb, int n_tok) {
     // With more tiles than CUs the most that any tail takes: a stream's scratch
     // reserved for a batch then also serves every smaller one of as many tiles.
-    if (split_tail && ceil_div(rows, TILE) * ceil_div(n_tok, TILE) > GEMM_CUS && nb - nb / GEMM_MAX_SPLITS >= GEMM_TAIL_BLOCKS)
-        return GEMM_CUS * PART;
-    const GemmShare s = gemm_share(rows, nb, n_tok, split_tail);
-    if (s.splits == 1) return 0;
-    return (size_t)s.splits * s.tail * PART;
+    return ceil_div(rows, TILE) * ceil_div(n_tok, TILE) > GEMM_CUS && nb - nb / GEMM_MAX_SPLITS >= GEMM_TAIL_BLOCKS
+               ? GEMM_TAIL_BYTES
+               : 0;
+}
+
+size_t gemm_workspace_bytes(int rows, int nb, int n_tok) {
+    const GemmShare s = gemm_share(rows, nb, n_tok);
+    if (s.full || s.splits == 1) return gemm_tail_bytes(rows, nb, n_tok);
+    return (size_t)s.splits * s.tail * GEMM_PART;
 }
 
 void launch_gemm_i8(int dtype, const uint8_t* qs, const float* swT, const int8_t* aq, const float* sxT, int rows,
-                    int nb, int n_tok, float* y, size_t y_stride, double* ws, bool split_tail, hipStream_t st) {
+                    int nb, int n_tok, float* y, size_t y_stride, double* ws, hipStream_t st) {
     GArgs g;
     g.qs = qs;
     g.swT = swT;
@@ -473,7 +479,7 @@ void launch_gemm_i8(int dtype, const uint8_t* qs, const float* swT, const int8_t
     g.n_tok = n_tok;
     g.tok_pad = gemm_tok_pad(n_tok);
     g.mtiles = ceil_div(n_tok, TILE);
-    const GemmShare sh = gemm_share(rows, nb, n_tok, split_tail);
+    const GemmShare sh = gemm_share(rows, nb, n_tok);
     g.full = sh.full;
     g.tail = sh.tail;
     g.splits = sh.splits;

@@ -1,7 +1,8 @@
 """The int8 GEMM where its tiles are not whole rounds of the CUs: the last round
 is split along K (one spare tile, half a round, rounds that the split does not
-take), against the exact sum of the quantized product; a capped scratch keeps the
-tail whole; and scratch reserved for a batch serves smaller ones under capture."""
+take), against the exact sum of the quantized product and the bits of a whole
+tile; the fixed-scratch call gives the ordinary call's bits; and scratch reserved for a
+batch serves smaller ones under capture."""
 import numpy as np
 import pytest
 
@@ -106,14 +107,35 @@ def test_split_tail_keeps_the_bits(dtype, rows, cols, n_tok, roll):
     wt.free()
 
 
-def test_capped_scratch_keeps_the_tail_whole():
-    """The fixed scratch (64 MiB) has no room for these activations and a split tail: the call is taken all the same."""
+def test_fixed_scratch_gives_the_same_bits():
+    """Activations that leave no room for the tail's parts in the fixed scratch
+    (64 MiB) are multiplied as by the ordinary call, also where a tail computed
+    whole would round otherwise: f32 groups 1, 2^-24, then 2^-54 each add up to
+    a tie in one f64 chain, and above it in the tail's parts."""
     import torch
-    rows, cols, n_tok = 30 * 128, 18944, 1100  # 270 tiles
+    rows, cols, n_tok = 30 * 128, 18944, 1100  # 270 tiles, 14 split
+    nb = cols // 32
     _, w = matrix(2, rows, cols, 5)
     x = torch.randn(n_tok, cols, device="cuda")
-    a, b = run(w, x), run(w, x, N.gemv_batch_dev_noalloc)
-    assert float((a.double() - b.double()).norm() / a.double().norm()) < 2e-7  # each within about 6e-8 of the exact sum
+    assert torch.equal(run(w, x), run(w, x, N.gemv_batch_dev_noalloc))
+    w.free()
+    q = np.zeros((rows, nb, 32), np.int8)
+    q[:, ::8, 1] = 1
+    s = np.full(nb, 2.0 ** -54, np.float32)
+    s[0], s[8] = 1, 2.0 ** -24
+    s = np.tile((s.view(np.uint32) >> 16).astype(np.uint16), (rows, 1))
+    w = N.Weight.q8_0(q.reshape(rows, cols), s.view(np.int16), rows, cols)
+    x = torch.zeros(n_tok, nb, 32, device="cuda")
+    x[..., 0], x[..., 1] = 127, 1  # scale 1, quants 127 and 1
+    x = x.view(n_tok, cols)
+    y = run(w, x)
+    assert torch.equal(y, run(w, x, N.gemv_batch_dev_noalloc))
+    assert bool((y[:, :28 * 128] == 1).all()) and bool((y[-50:, -128:] == 1 + 2.0 ** -23).all())
+    # What does not fit by itself is refused as before.
+    x, y = torch.zeros(2000, cols, device="cuda"), torch.empty(2000, rows, device="cuda")
+    w.prepare(N.ACT_I8, 2000)
+    with pytest.raises(N.InvalidArgument, match="no-alloc maximum"):
+        N.gemv_batch_dev_noalloc(w, x.data_ptr(), cols, y.data_ptr(), rows, 2000, N.ACT_I8)
     w.free()
 
 
