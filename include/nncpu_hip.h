@@ -322,7 +322,8 @@ int nnh_block_dots_dev(const nnh_weight* w, const void* act, size_t n_tok, int32
 
 /* Size the scratch of `stream` (and build the weight's layouts) for a call
  * (w, act, n_tok) ahead of time, so that such calls on `stream` allocate
- * nothing afterwards: for callers that capture them into a HIP graph, whose
+ * nothing afterwards, and neither do smaller batches whose layouts are built
+ * (nnh_weight_prepare): for callers that capture them into a HIP graph, whose
  * first call would otherwise grow the stream's scratch inside the capture.
  * No counterpart in the reference, whose scratch is per session
  * (model/kv.rs:324-332). */

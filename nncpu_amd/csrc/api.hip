@@ -13,6 +13,7 @@
 // mutex, synchronised), so a weight used in one mode holds only that mode's
 // copies.
 
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -299,7 +300,19 @@ size_t gemv_scratch_bytes(const nnh_weight* w, size_t n_tok, int act) {
     return act_layout(w->cols, n_tok, act).bytes + i8_workspace_bytes(w, n_tok, act);
 }
 
-// The part of it that the int8 GEMM's split tail takes.
+// The most that a call of up to n_tok vectors takes. The K splits follow from
+// the tile grid, so a smaller batch can need more: the largest of up to 16
+// vectors, and of each number of 128-vector tiles.
+size_t gemv_scratch_bytes_upto(const nnh_weight* w, size_t n_tok, int act) {
+    size_t most = n_tok ? gemv_scratch_bytes(w, std::min<size_t>(n_tok, GEMM_MIN_TOKENS - 1), act) : 0;
+    for (size_t n = 0; n < n_tok;) {
+        n = std::min(n + 128, n_tok);
+        most = std::max(most, gemv_scratch_bytes(w, n, act));
+    }
+    return most;
+}
+
+// The part of gemv_scratch_bytes that the int8 GEMM's split tail takes.
 size_t gemv_tail_bytes(const nnh_weight* w, size_t n_tok, int act) {
     if (w->dtype == NNH_BF16 || act != NNH_ACT_I8 || n_tok < GEMM_MIN_TOKENS) return 0;
     return nnh::gemm_tail_bytes((int)w->rows, (int)w->nb, (int)n_tok);
@@ -935,7 +948,7 @@ int nnh_stream_reserve(const nnh_weight* w, int act, size_t n_tok, void* stream)
     if (rc) return rc;
     if ((rc = check_call(w, 0, w ? w->rows : 0, n_tok, act))) return rc;
     if ((rc = prepare_locked(w, layouts_for(w, act, n_tok)))) return rc;
-    const size_t need = n_tok ? gemv_scratch_bytes(w, n_tok, act) : 0;
+    const size_t need = gemv_scratch_bytes_upto(w, n_tok, act);
     uint8_t* s = nullptr;
     if (need && (rc = scratch_locked((hipStream_t)stream, need, &s))) return rc;
     return NNH_OK;

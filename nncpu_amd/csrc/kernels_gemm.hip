@@ -451,18 +451,13 @@ GemmShare gemm_share(int rows, int nb, int n_tok) {
 constexpr size_t GEMM_PART = (size_t)TILE * TILE * sizeof(double);
 static_assert(GEMM_CUS * GEMM_PART == GEMM_TAIL_BYTES, "a split tail is at most one round of parts");
 
-size_t gemm_tail_bytes(int rows, int nb, int n_tok) {
-    // With more tiles than CUs the most that any tail takes: a stream's scratch
-    // reserved for a batch then also serves every smaller one of as many tiles.
-    return ceil_div(rows, TILE) * ceil_div(n_tok, TILE) > GEMM_CUS && nb - nb / GEMM_MAX_SPLITS >= GEMM_TAIL_BLOCKS
-               ? GEMM_TAIL_BYTES
-               : 0;
-}
-
 size_t gemm_workspace_bytes(int rows, int nb, int n_tok) {
     const GemmShare s = gemm_share(rows, nb, n_tok);
-    if (s.full || s.splits == 1) return gemm_tail_bytes(rows, nb, n_tok);
-    return (size_t)s.splits * s.tail * GEMM_PART;
+    return s.splits == 1 ? 0 : (size_t)s.splits * s.tail * GEMM_PART;
+}
+
+size_t gemm_tail_bytes(int rows, int nb, int n_tok) {
+    return gemm_share(rows, nb, n_tok).full ? gemm_workspace_bytes(rows, nb, n_tok) : 0;
 }
 
 void launch_gemm_i8(int dtype, const uint8_t* qs, const float* swT, const int8_t* aq, const float* sxT, int rows,

@@ -139,6 +139,29 @@ def test_fixed_scratch_gives_the_same_bits():
     w.free()
 
 
+@pytest.mark.parametrize("act", [1, 2])
+@pytest.mark.parametrize("rows,cols,n_tok", [
+    (170 * 128, 2048, 256),  # 340 tiles, 84 left in 3 parts; 128 vectors: 170 in 2 parts
+    (102 * 128, 3584, 400),  # 408 tiles, whole; 128 vectors: 102 in 3 parts
+])
+def test_reserved_scratch_holds_every_smaller_batch(act, rows, cols, n_tok):
+    import torch
+    _, w = matrix(1, rows, cols, 7)
+    x, y = torch.randn(n_tok, cols, device="cuda"), torch.empty(n_tok, rows, device="cuda")
+    st = torch.cuda.Stream()
+    w.prepare(act, 1).prepare(act, 16).prepare(act, n_tok)
+    N.stream_reserve(w, act, n_tok, st.cuda_stream)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    for n in (n_tok, 1, 5, 16, 17, 128, 129, n_tok - 1):
+        N.gemv_batch_dev(w, x.data_ptr(), cols, y.data_ptr(), rows, n, act, st.cuda_stream)
+        torch.cuda.synchronize()
+        # A scratch that grows at least doubles (60 MiB and more here); a kernel's first launch takes 2 MiB.
+        assert free - torch.cuda.mem_get_info()[0] < 16 << 20, n
+    N.stream_release(st.cuda_stream)
+    w.free()
+
+
 def test_reserved_stream_serves_smaller_batches_under_capture():
     import torch
     rows, cols = 86 * 128, 2048
