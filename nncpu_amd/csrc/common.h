@@ -163,6 +163,9 @@ void launch_gemv_f32(int dtype, const uint8_t* fq, const uint16_t* fs, const uin
 bool launch_gemm_f32(int dtype, const uint8_t* qs, const uint16_t* fs, const uint16_t* biases, const float* x,
                      size_t x_stride, float* xsum, int rows, int nb, int nbp, int n_tok, float* y, size_t y_stride,
                      bool v2, hipStream_t st);
+// Its split on `cus` CUs, and the most vectors of one launch (also BF16's).
+int batch_split(int rows, int n_tok, int cus);
+int batch_slice(int rows);
 
 // int8 path (kernels_i8.hip).
 void launch_quantize_act(const float* x, size_t x_stride, int cols, int n_tok, int8_t* q, uint16_t* s, double* sx,

@@ -678,26 +678,9 @@ void launch_bf16(BatchArgs g, hipStream_t st) {
     gemm_bf16_kernel<PATH, R, NT, NS><<<ceil_div(g.rows, 16 * R) * tiles, R * 256, LDS, st>>>(g);
 }
 
-// The split with the least time: rounds of workgroups over the CUs times a
-// workgroup's time per stage of 256 columns (us, measured for Q8_0 at 14336 and
-// 4096 rows; BF16's is within a tenth): 0 one row group and 16 vectors per
-// workgroup, 1 the same with a workgroup or less per CU, 2 two row groups and
-// 32 vectors, 3 two and 64.
-int pick_split(const BatchArgs& g) {
-    const int n16 = ceil_div(g.n_tok, 16), cus = cu_count();
-    const auto cost = [&](int r, int nt, double us) {
-        const long wgs = (long)ceil_div(g.rows, 16 * r) * ceil_div(n16, nt);
-        return (double)((wgs + cus - 1) / cus) * us;
-    };
-    const double c11 = cost(1, 1, 0.45), c22 = cost(2, 2, 1.42), c24 = cost(2, 4, 2.6);
-    if (c24 <= c11 && c24 <= c22) return 3;
-    if (c22 <= c11) return 2;
-    return (long)ceil_div(g.rows, 16) * n16 <= cus ? 1 : 0;
-}
-
 template <int DT>
 void launch_dt(const BatchArgs& g, hipStream_t st) {
-    switch (pick_split(g)) {
+    switch (batch_split(g.rows, g.n_tok, cu_count())) {
         case 1: launch_batch<DT, 1, 1, 2, 3>(g, st); break;
         case 0: launch_batch<DT, 1, 1, 1, 3>(g, st); break;
         case 2: launch_batch<DT, 2, 2, 1, 3>(g, st); break;
@@ -707,7 +690,7 @@ void launch_dt(const BatchArgs& g, hipStream_t st) {
 
 template <int PATH>
 void launch_path(const BatchArgs& g, hipStream_t st) {
-    switch (pick_split(g)) {
+    switch (batch_split(g.rows, g.n_tok, cu_count())) {
         case 0:
         case 1: launch_bf16<PATH, 1, 1, 3>(g, st); break;
         case 2: launch_bf16<PATH, 2, 2, 3>(g, st); break;
@@ -715,6 +698,43 @@ void launch_path(const BatchArgs& g, hipStream_t st) {
     }
 }
 
+}  // namespace
+
+// The split with the least time: rounds of workgroups over the CUs times a
+// workgroup's time per stage of 256 columns (us, measured for Q8_0 at 14336 and
+// 4096 rows; BF16's is within a tenth): 0 one row group and 16 vectors per
+// workgroup, 1 the same with a workgroup or less per CU, 2 two row groups and
+// 32 vectors, 3 two and 64.
+int batch_split(int rows, int n_tok, int cus) {
+    const int n16 = ceil_div(n_tok, 16);
+    const auto cost = [&](int r, int nt, double us) {
+        const long wgs = (long)ceil_div(rows, 16 * r) * ceil_div(n16, nt);
+        return (double)((wgs + cus - 1) / cus) * us;
+    };
+    const double c11 = cost(1, 1, 0.45), c22 = cost(2, 2, 1.42), c24 = cost(2, 4, 2.6);
+    if (c24 <= c11 && c24 <= c22) return 3;
+    if (c22 <= c11) return 2;
+    return (long)ceil_div(rows, 16) * n16 <= cus ? 1 : 0;
+}
+
+// Vectors of one launch: a grid holds less than 2^32 threads, and every split
+// has at most 512 per 16 rows x 16 vectors. 0: not even 16 vectors.
+int batch_slice(int rows) { return 16 * (int)(((size_t)1 << 22) / ceil_div(rows, 16)); }
+
+namespace {
+// g's vectors by slices; xsum, if any, has a row of nb per vector.
+template <class Launch>
+void launch_slices(const BatchArgs& g, const Launch& launch) {
+    const int step = batch_slice(g.rows);
+    for (long t = 0; t < g.n_tok; t += step) {
+        BatchArgs p = g;
+        p.x += (size_t)t * g.xs;
+        p.y += (size_t)t * g.ys;
+        if (p.xsum) p.xsum += (size_t)t * g.nb;
+        p.n_tok = (int)(g.n_tok - t < step ? g.n_tok - t : step);
+        launch(p);
+    }
+}
 }  // namespace
 
 bool launch_gemm_f32(int dtype, const uint8_t* qs, const uint16_t* fs, const uint16_t* biases, const float* x,
@@ -727,14 +747,18 @@ bool launch_gemm_f32(int dtype, const uint8_t* qs, const uint16_t* fs, const uin
     // 48.4; Q4 14336 x 4096 four 38.0 / 38.0, six 60.8 / 38.4.
     if (n_tok < (dtype == 1 ? (v2 ? 3 : 2) : (v2 ? 5 : 3))) return false;
     // 16-byte pieces of x; 32-bit byte offsets within a tile's rows.
-    if (((uintptr_t)x & 15) || (x_stride & 3) || x_stride >= ((size_t)1 << 23) || nb >= (1 << 21)) return false;
+    if (((uintptr_t)x & 15) || (x_stride & 3) || x_stride >= ((size_t)1 << 23) || nb >= (1 << 21) ||
+        batch_slice(rows) == 0)
+        return false;
     if (dtype == 2) launch_block_sums(x, x_stride, nb, n_tok, xsum, st);
     const BatchArgs g{qs, fs,       biases, x,  xsum, y, x_stride, y_stride,
                       rows, nb, nbp, n_tok, 0, 0, 0, 0, ((uintptr_t)y & 15) == 0 && (y_stride & 3) == 0};
-    if (dtype == 1)
-        launch_dt<1>(g, st);
-    else
-        launch_dt<2>(g, st);
+    launch_slices(g, [&](const BatchArgs& p) {
+        if (dtype == 1)
+            launch_dt<1>(p, st);
+        else
+            launch_dt<2>(p, st);
+    });
     return true;
 }
 
@@ -743,16 +767,18 @@ bool launch_gemm_bf16(int path, const uint16_t* raw, int rows, int cols, const f
     // Few vectors stay on the chain kernel: measured, that against here, three
     // vectors 6144 x 1536 8.0 / 8.3 us, 14336 x 4096 34.1 / 33.8, four 10.0 / 8.3.
     if (path == BF16_PATH_F64 || n_tok < 4 || ((uintptr_t)x & 15) || (x_stride & 3) ||
-        x_stride >= ((size_t)1 << 23) || cols >= (1 << 26))
+        x_stride >= ((size_t)1 << 23) || cols >= (1 << 26) || batch_slice(rows) == 0)
         return false;
     const BatchArgs g{(const uint8_t*)raw, nullptr, nullptr, x, nullptr, y, x_stride, y_stride, rows, cols / 32, 0, n_tok,
                       cols % 32,           0,       0,       0, ((uintptr_t)y & 15) == 0 && (y_stride & 3) == 0};
-    if (path == BF16_PATH_QUAD)
-        launch_path<BF16_PATH_QUAD>(g, st);
-    else if (path == BF16_PATH_ROW8)
-        launch_path<BF16_PATH_ROW8>(g, st);
-    else
-        launch_path<BF16_PATH_ROW32>(g, st);
+    launch_slices(g, [&](const BatchArgs& p) {
+        if (path == BF16_PATH_QUAD)
+            launch_path<BF16_PATH_QUAD>(p, st);
+        else if (path == BF16_PATH_ROW8)
+            launch_path<BF16_PATH_ROW8>(p, st);
+        else
+            launch_path<BF16_PATH_ROW32>(p, st);
+    });
     return true;
 }
 

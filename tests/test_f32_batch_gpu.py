@@ -86,3 +86,28 @@ def test_bf16_batch_bit_exact(oracle, rows, cols, n_tok, pad):
         got = y[t * ys:t * ys + rows]
         assert np.array_equal(got.view(np.uint32), want[t * ys:t * ys + rows].view(np.uint32)), t
     wt.free()
+
+
+@pytest.mark.parametrize("fmt", ["q8", "q4", "bf16"])
+def test_more_vectors_than_one_launch_holds(fmt):
+    """65552 rows take 16368 vectors a launch: those around the slice's end as alone."""
+    import torch
+    rows, cols, n_tok, edge = 65552, 32, 16400, 16368
+    rng = np.random.default_rng(9)
+    s = (rng.uniform(1e-2, 2e-2, (rows, 1)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16).view(np.int16)
+    if fmt == "q8":
+        w = N.Weight.q8_0(rng.integers(-127, 128, (rows, cols), dtype=np.int8), s, rows, cols)
+    elif fmt == "q4":
+        w = N.Weight.q4(rng.integers(0, 256, (rows, cols // 2), dtype=np.uint8), s, s, rows, cols)
+    else:
+        w = N.Weight.bf16((rng.standard_normal((rows, cols)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16),
+                          rows, cols)
+    x, y = torch.randn(n_tok, cols, device="cuda"), torch.full((n_tok, rows), 7.0, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    w.prepare(N.ACT_F32, n_tok)
+    N.gemv_batch_dev(w, x.data_ptr(), cols, y.data_ptr(), rows, n_tok, N.ACT_F32, st)
+    few = torch.full((16, rows), 7.0, device="cuda")
+    for t in (0, edge - 16, edge, n_tok - 16):
+        N.gemv_batch_dev(w, x[t:].data_ptr(), cols, few.data_ptr(), rows, 16, N.ACT_F32, st)
+        assert torch.equal(y[t:t + 16], few), t
+    w.free()
