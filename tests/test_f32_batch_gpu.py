@@ -88,6 +88,41 @@ def test_bf16_batch_bit_exact(oracle, rows, cols, n_tok, pad):
     wt.free()
 
 
+# The splits of two row groups, by the number of 16-vector groups in a token
+# tile: 32 vectors at most (a full tile; tiles of two and one), 64 at most in a
+# ring of two stages (tiles of three; of four and three; of four), each with
+# a ragged last row tile, and stages that are whole or not.
+LARGE = [(6163, 17, 2), (2470, 75, 2), (6841, 33, 3), (2934, 103, 3), (5141, 64, 3)]
+
+
+def split_of(rows, n_tok):
+    import torch
+    f = N.lib()._ZN3nnh11batch_splitEiii  # nnh::batch_split(int rows, int n_tok, int cus)
+    return f(rows, n_tok, torch.cuda.get_device_properties(0).multi_processor_count)
+
+
+@pytest.mark.parametrize("dtype", [1, 2])
+@pytest.mark.parametrize("cols", [96, 544, 1024, 1312])
+@pytest.mark.parametrize("rows,n_tok,split", LARGE)
+def test_f32_batch_large_splits(oracle, dtype, rows, cols, n_tok, split):
+    assert split_of(rows, n_tok) == split
+    pad = 4 * (n_tok & 1)
+    rng = np.random.default_rng(rows + cols)
+    x = np.ldexp(rng.standard_normal(n_tok * (cols + pad)), rng.integers(-140, 60, n_tok * (cols + pad))).astype(np.float32)
+    x[rng.integers(0, x.size, x.size // 8)] = -0.0
+    y, ref = run(oracle, dtype, rows, cols, n_tok, pad, x=x)
+    assert np.array_equal(y.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("path,cols", [("quad", 24), ("quad", 1304), ("quad", 512), ("row8", 264), ("row8", 1304),
+                                       ("row32", 96), ("row32", 1312), ("row32", 768)])
+@pytest.mark.parametrize("rows,n_tok,split", LARGE)
+def test_bf16_batch_large_splits(oracle, path, rows, cols, n_tok, split):
+    rows = (rows + 3) // 4 * 4 if path == "quad" else rows | 1
+    assert split_of(rows, n_tok) == split
+    test_bf16_batch_bit_exact(oracle, rows, cols, n_tok, 4 * (n_tok & 1))
+
+
 @pytest.mark.parametrize("fmt", ["q8", "q4", "bf16"])
 def test_more_vectors_than_one_launch_holds(fmt):
     """65552 rows take 16368 vectors a launch: those around the slice's end as alone."""
