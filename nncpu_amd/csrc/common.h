@@ -166,6 +166,9 @@ bool launch_gemm_f32(int dtype, const uint8_t* qs, const uint16_t* fs, const uin
 // Its split on `cus` CUs, and the most vectors of one launch (also BF16's).
 int batch_split(int rows, int n_tok, int cus);
 int batch_slice(int rows);
+// Whether a few vectors are taken here, by measured times.
+bool batch_wins(int dtype, int rows, int nb, int n_tok, bool v2);
+bool batch_wins_bf16(int path, int rows, int cols, int n_tok);
 
 // int8 path (kernels_i8.hip).
 void launch_quantize_act(const float* x, size_t x_stride, int cols, int n_tok, int8_t* q, uint16_t* s, double* sx,

@@ -721,6 +721,61 @@ int batch_split(int rows, int n_tok, int cus) {
 // has at most 512 per 16 rows x 16 vectors. 0: not even 16 vectors.
 int batch_slice(int rows) { return 16 * (int)(((size_t)1 << 22) / ceil_div(rows, 16)); }
 
+// Few vectors: a group of 16 costs the same from 1 to 16, in rounds of 16 rows
+// per CU, so short rows, a partial round and many rounds of two to eight vectors
+// are left to the kernels of kernels_f32.hip (one vector at a time, or four at
+// a time through the tall matrices' kernel). Measured, both at 2000 sizes from
+// 128 x 512 to 151936 x 512 and 28672 x 4096; us, those against these: Q8_0 two
+// vectors 4096 x 4096 11.7 / 10.4, 256 x 4096 9.1 / 10.1, 2048 x 12288 22.1 /
+// 24.8, three 20000 x 1024 10.1 / 13.2, 28672 x 4096 58.6 / 47.4; Q4 three
+// 4096 x 4096 15.7 / 15.0, 8192 x 1024 9.6 / 10.5, five 65536 x 1024 41.2 / 60.8,
+// 14336 x 4096 45.4 / 36.1.
+bool batch_wins(int dtype, int rows, int nb, int n_tok, bool v2) {
+    if (n_tok > 12) return true;
+    if (v2) {
+        // The blocks per row from which these are no slower, by vectors and rows.
+        constexpr short NO = 32767;
+        constexpr int ROWS[5] = {12288, 16384, 24576, 32767, 49152};
+        constexpr short MIN[2][6][6] = {
+            {{48, 216, 216, 216, 216, 216},  // Q8_0: 2 vectors
+             {48, 80, 171, 112, 171, 171},   // 3
+             {48, 48, 112, 112, 144, 144},   // 4
+             {0, 0, 32, 32, 0, 48},          // 5, 6
+             {0, 0, 0, 0, 0, 32},            // 7, 8
+             {0, 0, 0, 0, 0, 0}},            // 9 .. 12
+            {{NO, NO, NO, NO, NO, NO},     // Q4
+             {NO, NO, NO, NO, NO, NO},
+             {NO, NO, NO, NO, NO, NO},
+             {32, 48, 80, 112, 48, 112},
+             {0, 32, 48, 64, 32, 80},
+             {0, 0, 0, 0, 0, 32}}};
+        int c = 0;
+        while (c < 5 && rows > ROWS[c]) ++c;
+        return nb >= MIN[dtype - 1][n_tok <= 4 ? n_tok - 2 : n_tok <= 6 ? 3 : n_tok <= 8 ? 4 : 5][c];
+    }
+    if (dtype == 1) {
+        if (n_tok > 2) return true;
+        if (rows < 2048) return nb <= 80 || nb > 256 || (rows >= 1280 && nb <= 128);
+        if (rows <= 4096) return nb <= 48 || (rows >= 2560 && nb <= 96) || rows >= 3584;
+        if (rows <= 8192) return nb <= 24 || rows >= 7168;
+        return rows >= 11776 && nb >= 64;
+    }
+    if (n_tok > 4) return true;
+    if (n_tok == 4) return rows <= 4096 || (rows <= 8192 ? nb >= 24 && (rows >= 6144 || nb < 384) : nb >= 48);
+    if (n_tok < 3 || nb <= 32) return false;
+    if (rows <= 4096) return rows < 2048 || nb <= 160 || rows >= 3584;
+    return nb >= 64 && rows >= 7168;
+}
+
+// BF16: measured likewise (four vectors, us): 256 x 4096 15.8 / 12.4, 257 x 4096
+// 8.2 / 10.9, 4097 x 4096 22.8 / 15.0, 14336 x 2048 13.5 / 18.3, x 4096 37.8 / 31.4;
+// from five no size was slower.
+bool batch_wins_bf16(int path, int rows, int cols, int n_tok) {
+    if (n_tok != 4) return n_tok > 4;
+    if (path == BF16_PATH_ROW32) return cols < 2048 || (rows > 2048 ? cols >= 4096 || rows > 3000 : cols > 8192);
+    return rows <= 8192 || cols >= 4096 || (path == BF16_PATH_ROW8 && cols <= 520);
+}
+
 namespace {
 // g's vectors by slices; xsum, if any, has a row of nb per vector.
 template <class Launch>
@@ -740,12 +795,7 @@ void launch_slices(const BatchArgs& g, const Launch& launch) {
 bool launch_gemm_f32(int dtype, const uint8_t* qs, const uint16_t* fs, const uint16_t* biases, const float* x,
                      size_t x_stride, float* xsum, int rows, int nb, int nbp, int n_tok, float* y, size_t y_stride,
                      bool v2, hipStream_t st) {
-    // A group of 16 vectors costs the same from 1 to 16, so a few go through
-    // the one-vector or (tall, v2) few-vector kernels. Measured, these against
-    // here: two vectors Q8 4096 x 4096 12.2 / 10.8 us, 14336 x 4096 (tall) 27.0
-    // / 30.6; Q4 4096 x 4096 11.3 / 14.9, three 16.6 / 15.0, 3584 x 18944 48.1 /
-    // 48.4; Q4 14336 x 4096 four 38.0 / 38.0, six 60.8 / 38.4.
-    if (n_tok < (dtype == 1 ? (v2 ? 3 : 2) : (v2 ? 5 : 3))) return false;
+    if (n_tok < 2 || !batch_wins(dtype, rows, nb, n_tok, v2)) return false;
     // 16-byte pieces of x; 32-bit byte offsets within a tile's rows.
     if (((uintptr_t)x & 15) || (x_stride & 3) || x_stride >= ((size_t)1 << 23) || nb >= (1 << 21) ||
         batch_slice(rows) == 0)
@@ -764,9 +814,7 @@ bool launch_gemm_f32(int dtype, const uint8_t* qs, const uint16_t* fs, const uin
 
 bool launch_gemm_bf16(int path, const uint16_t* raw, int rows, int cols, const float* x, size_t x_stride, int n_tok,
                       float* y, size_t y_stride, hipStream_t st) {
-    // Few vectors stay on the chain kernel: measured, that against here, three
-    // vectors 6144 x 1536 8.0 / 8.3 us, 14336 x 4096 34.1 / 33.8, four 10.0 / 8.3.
-    if (path == BF16_PATH_F64 || n_tok < 4 || ((uintptr_t)x & 15) || (x_stride & 3) ||
+    if (path == BF16_PATH_F64 || !batch_wins_bf16(path, rows, cols, n_tok) || ((uintptr_t)x & 15) || (x_stride & 3) ||
         x_stride >= ((size_t)1 << 23) || cols >= (1 << 26) || batch_slice(rows) == 0)
         return false;
     const BatchArgs g{(const uint8_t*)raw, nullptr, nullptr, x, nullptr, y, x_stride, y_stride, rows, cols / 32, 0, n_tok,
