@@ -95,6 +95,8 @@ __device__ __forceinline__ int mx_exponent(float amax) {
 // and 1 to 2 us slower at 1024 to 3584 (too few waves). Quantizing and
 // multiplying by a 256-row Q8_0 matrix, us, with a lane per value and now: 512
 // tokens of 3584 32.4 / 28.3, 512 of 18944 72.7 / 48.6, 17 of 2048 23.8 / 23.8.
+// The quantizer alone, all parts, 8 tokens of 1152 2.9 / 3.1, of 3584 3.6 / 3.2, of
+// 18944 9.9 / 5.0 (3.4, 3.6 and 8.1 when padding was computed like tokens).
 // Blocks past nb (up to the group-padded nbp8) and tokens past n_tok (up to
 // xl_tok, whole GEMM token tiles) only write zeros: the limbs of xl, and for
 // tokens past n_tok the xb values. PARTS: which parts of the buffer are written
@@ -111,12 +113,17 @@ __global__ __launch_bounds__(256) void quantize_mx_kernel(const float* __restric
     const int nb = cols >> 5, p = threadIdx.x & 7, grp = threadIdx.x >> 3;
     const int gx = nbp8 >> 2;  // workgroups along the blocks (one-dimensional grid: any number of vectors)
     const int t = blockIdx.x / gx * 8 + (grp & 7), b = blockIdx.x % gx * 4 + (grp >> 3);  // xl_tok, nbp8: multiples of 8
-    const f4u v = *(const f4u*)(x + (size_t)(t < n_tok ? t : n_tok - 1) * x_stride + 32 * (size_t)(b < nb ? b : nb - 1) +
-                                4 * p);  // in bounds
     // xb tiled: [token tile][block][token in tile][32], 16-byte chunks of a
     // row swizzled as the GEMM's LDS rows are (chunk c at c ^ ((row >> 2) & 3)).
     const int tt = t / MX_TM_Q, tr = t % MX_TM_Q;
     uint16_t* xw = xb + ((size_t)tt * nb * MX_TM_Q + tr) * 32 + (((p >> 1) ^ ((tr >> 2) & 3)) << 3) + 4 * (p & 1);
+    if (GEMM && t - (grp & 7) >= n_tok) {  // a workgroup of padding (most of them where few tokens fill a tile): zeros
+        if (b < nb) *(uint2*)(xw + (size_t)b * MX_TM_Q * 32) = uint2{0, 0};
+        if (p == 0) *(uint32_t*)(xl + ((size_t)t * nbp8 + b) * 2) = 0;
+        return;
+    }
+    const f4u v = *(const f4u*)(x + (size_t)(t < n_tok ? t : n_tok - 1) * x_stride + 32 * (size_t)(b < nb ? b : nb - 1) +
+                                4 * p);  // in bounds
     // amax over the block, NaN skipped (as nncpu's encoder's `v.abs() > amax`).
     const float a = max8(fmaxf(fmaxf(q8_abs(v[0]), q8_abs(v[1])), fmaxf(q8_abs(v[2]), q8_abs(v[3]))));
     const bool zero = !(a > 0.0f);
