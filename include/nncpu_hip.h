@@ -221,7 +221,11 @@ int nnh_model_argmax_dev(const nnh_weight* w, const float* x, float* logits, voi
  * threads (lib.rs:36-41). A buffer that has to grow is replaced, and the old
  * one is kept until the process ends, so a call captured in a HIP graph stays
  * valid after larger calls; replays of graphs captured on the same stream
- * share that stream's scratch, so they must not overlap each other. */
+ * share that stream's scratch, so they must not overlap each other. Any
+ * alignment of x is taken, with the same bits; several vectors on f32
+ * activations are fastest with x 16-byte aligned and x_stride a multiple of 4
+ * (other rows go through kernels of up to four vectors at a time: 301 vectors
+ * of a 14336 x 4096 matrix 2.7 ms against 0.35). */
 int nnh_gemv_batch_dev(const nnh_weight* w, const float* x, size_t x_stride, float* y, size_t y_stride,
                        size_t n_tok, int act, void* stream);
 

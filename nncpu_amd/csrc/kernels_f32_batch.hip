@@ -28,7 +28,8 @@
 //
 // Data moves global -> LDS directly (no registers) through a ring of NS
 // stages of 8 blocks. 16-byte pieces are XOR-swizzled by row on the global
-// side, so every LDS read is spread over all banks. Weights come from the
+// side, so that LDS reads are spread over the banks (the LDS is active 16 to 18 %
+// of the time, a quarter to a half of that in conflicts). Weights come from the
 // split layout as uploaded, scales from the f32 path's padded rows (16 bytes
 // are 8 blocks). In a partial last stage the missing blocks are 0 * -0 = -0,
 // which leaves every accumulator as it is, -0 included.

@@ -394,7 +394,10 @@ __device__ __forceinline__ int tok_blocks(const AttnArgs& a, int p0, int n_seq, 
 // head). Qwen2.5-7B shape (28 / 4 heads of 128), 512
 // tokens: 51 us per layer, 123 with the FMAs on the vector unit fed from LDS
 // (4 bytes of LDS return per FMA); with tokens of one block finished here, the
-// merge after it 15 -> 12.
+// merge after it 15 -> 12. Both kernels at other shapes: 17 tokens 40 -> 18, 14 / 2
+// heads of 64, 512 tokens 58 -> 30, 4 / 1 of 256 112 -> 37; least where a tile holds
+// 32 tokens of one head under a short window, whose keys are mostly edges (8 / 8
+// heads of 128, window 64: 97 -> 87).
 constexpr int AT_NQ = 32;   // rows per workgroup at most (16 at head_dim 256: registers)
 constexpr int AT_CUS = 256;  // CUs of the GPU (workgroup order only)
 constexpr int AT_SC = ATTN_BLOCK + 4;  // floats per LDS row: rows 4 apart fall on other banks
