@@ -88,6 +88,29 @@ def test_bf16_batch_bit_exact(oracle, rows, cols, n_tok, pad):
     wt.free()
 
 
+@pytest.mark.parametrize("rows,cols", [(48, 520), (51, 520), (51, 544)])  # the 4-row, the 8- and the 32-chain kernel's
+def test_bf16_batch_special_values(oracle, rows, cols):
+    n_tok = 19
+    rng = np.random.default_rng(rows + cols)
+    w = oracle.f32_array_to_bf16(np.ldexp(rng.standard_normal(rows * cols), rng.integers(-140, 20, rows * cols)).astype(np.float32))
+    w[rng.integers(0, w.size, w.size // 8)] = 0x8000
+    w[7 * cols + 3], w[9 * cols + cols - 1], w[11 * cols + 40] = 0x7F80, 0x7FC0, 1
+    x = np.ldexp(rng.standard_normal(n_tok * cols), rng.integers(-150, 100, n_tok * cols)).astype(np.float32)
+    x[rng.integers(0, x.size, x.size // 8)] = -0.0
+    x.reshape(n_tok, cols)[3] = -0.0
+    x.reshape(n_tok, cols)[5, -1] = np.inf
+    x.reshape(n_tok, cols)[6, 40] = 3e38
+    x.reshape(n_tok, cols)[7, 5] = np.nan
+    wt = N.Weight.bf16(w, rows, cols)
+    y = np.zeros(n_tok * rows, np.float32)
+    N.gemv_batch(wt, x, cols, y, rows, n_tok)
+    ref = oracle.gemv_bf16(w, x, rows, cols, n_tok, cols, rows)
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(y), nan) and nan.reshape(n_tok, rows)[7].all() and not nan.all()
+    assert np.array_equal(y[~nan].view(np.uint32), ref[~nan].view(np.uint32))
+    wt.free()
+
+
 # The splits of two row groups, by the number of 16-vector groups in a token
 # tile: 32 vectors at most (a full tile; tiles of two and one), 64 at most in a
 # ring of two stages (tiles of three; of four and three; of four), each with
