@@ -55,7 +55,7 @@ def faults(code):
     return copies, m0, base
 
 
-def test_checker_sees_both_hazards():
+def test_scan_sees_both_hazards():
     code = ["0000 <k>:", "\ts_mov_b32 m0, s1", "\tglobal_load_lds_dwordx4 v1, s[2:3]",
             "\ts_mov_b32 m0, s1", "\ts_nop 0", "\tglobal_load_lds_dwordx4 v1, s[2:3]",
             "\tv_readfirstlane_b32 s2, v0", "\ts_nop 3", "\tglobal_load_lds_dwordx4 v1, s[2:3]",
