@@ -28,7 +28,10 @@ namespace {
 //     the block-major scales are written in runs; from QUANT_TILE_MIN vectors.
 //     (Four blocks a lane, whose loads would be in flight together, leave too few
 //     waves: 1.0 to 2.8 us more at 17 to 512 vectors of 1024 to 18944.)
-//   otherwise a wave takes 8 consecutive blocks; few vectors.
+//   otherwise a wave takes 8 consecutive blocks and is a workgroup; few vectors
+//     (four waves a workgroup kept the few blocks on fewer CUs: quantizing 8 of
+//     1024 and multiplying by 256 rows in a graph 8.07 us, 7.79 now, 7.89 with a
+//     lane per value; 8 of 6144 by 1536 rows 9.92, 9.85, 9.93).
 // Quantizing and multiplying by a 256-row Q8_0 matrix, us, with a lane per value
 // and now: 17 vectors of 2048 21.2 / 21.0, 512 of 3584 34.6 / 30.3, 512 of 18944
 // 79.6 / 59.6.
@@ -47,7 +50,7 @@ __global__ __launch_bounds__(256) void quantize_act_kernel(const float* __restri
         t = blockIdx.x / gx * 8 + (grp & 7);
         b = blockIdx.x % gx * 4 + (grp >> 3);
     } else {
-        const int blk = blockIdx.x * 32 + grp;
+        const int blk = blockIdx.x * 8 + grp;
         t = blk / nb;
         b = blk - t * nb;
     }
@@ -982,7 +985,7 @@ void launch_quantize_act(const float* x, size_t x_stride, int cols, int n_tok, i
         quantize_act_kernel<true><<<ceil_div(nb, 4) * ceil_div(n_tok, 8), 256, 0, st>>>(x, x_stride, cols, n_tok, q, s, sx,
                                                                                         sxT, tok_pad);
     else
-        quantize_act_kernel<false><<<ceil_div((long)nb * n_tok, 32), 256, 0, st>>>(x, x_stride, cols, n_tok, q, s, sx,
+        quantize_act_kernel<false><<<ceil_div((long)nb * n_tok, 8), 64, 0, st>>>(x, x_stride, cols, n_tok, q, s, sx,
                                                                                    sxT, tok_pad);
 }
 
